@@ -159,6 +159,9 @@ __device__ __forceinline__ int block_class_rank(int k, int (&tot)[NCH]) {
 
 // Pass 1: classify and count per block.  Blocks [0, nbu) take the unique rows, blocks [nbu, nbu + nbd) the dynamic
 // slots.  Block counts go channel-major: bu[c * nbu + b], bd[c * nbd + b]; bbad[b]: the block's rows outside [0, R).
+// badm (the device-driven step, else NULL): badm[b] and badm[nbu + b] count the block's admitted rows that appear in
+// the next batches and those that do not, by the class each takes if it is not admitted after all (drop_target),
+// kAdmBits bits per class in one word.  The overflow path (plan_overflow) then needs no pass over the rows.
 struct PlanCount {
   elr_plan_in p;
   elr_plan_out o;
@@ -166,13 +169,34 @@ struct PlanCount {
   int64_t* bu;
   int64_t* bd;
   int64_t* bbad;
+  int64_t* badm;
   __device__ void operator()(int64_t b, int64_t) const;
 };
+
+// The classes an admitted row takes when the overflow path drops its admission (srm2/elara.py:250-251), as targets
+// 0..4: N append, N compact, L append, L compact, and (F rows) transient or S.
+constexpr int kDropTargets = 5;
+constexpr int kAdmBits = 12;   // a block's count is at most kPlanBlock
+static_assert(kPlanBlock < (1 << kAdmBits) && kDropTargets * kAdmBits < 64, "a block's counts fit in one word");
+
+__device__ __forceinline__ int drop_target(int f) {
+  return (f & ELR_PLAN_N) ? ((f & ELR_PLAN_APP) ? 0 : 1) : (f & ELR_PLAN_L) ? ((f & ELR_PLAN_APP) ? 2 : 3) : 4;
+}
+__device__ __forceinline__ int adm_field(int64_t w, int t) { return (int)(w >> (kAdmBits * t)) & ((1 << kAdmBits) - 1); }
+__device__ __forceinline__ int adm_total(int64_t w) {
+  int n = 0;
+#pragma unroll
+  for (int t = 0; t < kDropTargets; ++t) n += adm_field(w, t);
+  return n;
+}
 
 __device__ void PlanCount::operator()(int64_t b, int64_t) const {
   if (b < nbu) {
     __shared__ int nbad;
+    __shared__ unsigned long long nadm[2];
     if (threadIdx.x == 0) nbad = 0;
+    if (threadIdx.x < 2) nadm[threadIdx.x] = 0;
+    int fl = 0;
     const int64_t i = b * kPlanBlock + threadIdx.x;
     int k = -1;
     bool bad = false;
@@ -181,18 +205,22 @@ __device__ void PlanCount::operator()(int64_t b, int64_t) const {
       const RowClass rc = classify_row(p, r);
       bad = !row_ok(p, r);
       k = kRankOf[rc.cls];
+      fl = rc.flags;
       o.cls[i] = (int8_t)rc.cls;
       o.flags[i] = (uint8_t)rc.flags;
       o.sl[i] = rc.sl;
       o.c[i] = (int8_t)rc.c;
     }
     int tot[kNumCls];
-    block_class_rank<kNumCls>(k, tot);   // synchronises the block: nbad is zeroed before the adds below
+    block_class_rank<kNumCls>(k, tot);   // synchronises the block: nbad and nadm are zeroed before the adds below
+    if (badm && (fl & ELR_PLAN_ADMIT))
+      atomicAdd(&nadm[(fl & ELR_PLAN_NEXT) ? 0 : 1], 1ull << (kAdmBits * drop_target(fl)));
     const uint64_t mb = __builtin_amdgcn_ballot_w64(bad);
     if ((threadIdx.x & 63) == 0 && mb) atomicAdd(&nbad, (int)__builtin_popcountll(mb));
     if (threadIdx.x < kNumCls) bu[threadIdx.x * nbu + b] = tot[threadIdx.x];
     __syncthreads();
     if (threadIdx.x == 0) bbad[b] = nbad;
+    if (badm && threadIdx.x < 2) badm[threadIdx.x * nbu + b] = (int64_t)nadm[threadIdx.x];
   } else {
     const int64_t bb = b - nbu;
     const int64_t j = bb * kPlanBlock + threadIdx.x;
@@ -211,84 +239,120 @@ __device__ void PlanCount::operator()(int64_t b, int64_t) const {
 // ---- the device-driven step's resolution (elr_plan_step) ------------------------------------------------------
 constexpr int kRW = kScanBlock / 64;   // waves of the resolving block
 
-// The overflow path (srm2/elara.py:246-256) by the resolving block: the admitted rows are ordered as the reference's
-// stable sort of pri = (admitted and in the next batches: 0, admitted otherwise: 2) orders them, the last `need` of
-// them are not admitted after all and take the class they get without admission (their cls is rewritten), and the
-// class-rank block offsets and totals are recomputed into bu2 and tot2 (exclusive offsets per block of kPlanBlock
-// rows, as the scan launch makes them).  Returns, to thread 0, how many dropped rows appear in the next batches.
+// What the overflow path drops (srm2/elara.py:246-256).  The reference's stable sort of pri = (admitted and in the
+// next batches: 0, admitted otherwise: 2) ranks the admitted rows of the next batches first and the other admitted rows
+// after them, each in row order, and the last `need` are not admitted after all.  That is one row position: with
+// `all` the admitted rows outside the next batches are dropped, and of the others those at or past `cut`; without
+// it only rows outside the next batches at or past `cut`.
+struct DropCut {
+  int64_t all, cut;
+};
+__device__ __forceinline__ bool dropped(const DropCut& c, int f, int64_t i) {
+  if (!(f & ELR_PLAN_ADMIT)) return false;
+  return (f & ELR_PLAN_NEXT) ? (c.all && i >= c.cut) : (c.all || i >= c.cut);
+}
+// The class of a dropped row.
+__device__ __forceinline__ int drop_class(int f, int want_t) {
+  const int t = drop_target(f);
+  return t == 0 ? kNApp : t == 1 ? kNCmp : t == 2 ? kLApp : t == 3 ? kLCmp : (want_t ? kFNAdm : kS);
+}
+
+// The overflow path by the resolving block: the cut from the blocks' counts of admitted rows (badm) and the rows of
+// the one block it falls in, then the class-rank block offsets and totals with the dropped rows in their new classes,
+// into bu2 and tot2 (bu: the offsets without the drops).  The scatter launch reclassifies the dropped rows.  It walks
+// counts and not rows: at 119k unique rows (464 blocks) the launch takes 16.6 us with an overflow, against 269 for a
+// loop over the rows in this block.  Returns, to thread 0, how many dropped rows appear in the next batches.
 __device__ int64_t plan_overflow(const elr_plan_in& p, const elr_plan_out& o, int64_t n, int64_t nbu, int64_t n_adm,
-                                 int64_t need, int64_t* __restrict__ bu2, int64_t* __restrict__ tot2) {
-  __shared__ int64_t a0_w[kRW];
-  __shared__ int wsum[kRW][3];
-  __shared__ int wcls[kRW][kNumCls];
-  __shared__ int64_t run[kNumCls + 3];   // class runs, then admitted rows in / not in the next batches, carry drops
+                                 int64_t need, const int64_t* bu, const int64_t* tot, const int64_t* badm,
+                                 int64_t* bu2, int64_t* tot2, DropCut* out_cut) {
+  __shared__ int64_t wsum[kRW];
+  __shared__ int64_t cut_blk, cut_rank, cut_row;
+  __shared__ unsigned long long cut_pack;   // the cut's block: its dropped rows by target
+  __shared__ int wcnt[kPlanBlock / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // admitted rows that appear in the next batches: they come first in the reference's priority order
+  const int64_t live = (n + kPlanBlock - 1) / kPlanBlock, nb = live < nbu ? live : nbu;
+  // A0: the admitted rows of the next batches
   int64_t a0 = 0;
-  for (int64_t i = threadIdx.x; i < n; i += kScanBlock) {
-    const int f = o.flags[i];
-    a0 += ((f & ELR_PLAN_ADMIT) && (f & ELR_PLAN_NEXT)) ? 1 : 0;
-  }
+  for (int64_t b = threadIdx.x; b < nb; b += kScanBlock) a0 += adm_total(badm[b]);
   a0 = wave_incl_scan<int64_t>(a0);
-  if (lane == 63) a0_w[w] = a0;
-  if (threadIdx.x < kNumCls + 3) run[threadIdx.x] = 0;
+  if (lane == 63) wsum[w] = a0;
+  if (threadIdx.x == 0) {
+    cut_blk = nb;
+    cut_rank = 0;
+    cut_row = n;
+    cut_pack = 0;
+  }
   __syncthreads();
   int64_t A0 = 0;
-  for (int v = 0; v < kRW; ++v) A0 += a0_w[v];
+  for (int v = 0; v < kRW; ++v) A0 += wsum[v];
   const int64_t T = n_adm - need;   // admitted rows at priority rank T and beyond are dropped
-  for (int64_t c0 = 0; c0 < n; c0 += kScanBlock) {
-    const int64_t i = c0 + threadIdx.x;
-    const bool valid = i < n;
-    const int f = valid ? o.flags[i] : 0;
-    const bool adm = (f & ELR_PLAN_ADMIT) != 0, nx = (f & ELR_PLAN_NEXT) != 0;
-    const uint64_t m_nx = __builtin_amdgcn_ballot_w64(adm && nx), m_x = __builtin_amdgcn_ballot_w64(adm && !nx);
-    if (lane == 0) {
-      wsum[w][0] = __builtin_popcountll(m_nx);
-      wsum[w][1] = __builtin_popcountll(m_x);
-    }
+  const bool all = T < A0;
+  const int64_t rank = all ? T : T - A0;                       // the cut row's rank in its list
+  const int64_t* list = badm + (all ? 0 : nbu);   // the list the cut falls in
+  int64_t run = 0;
+  for (int64_t c0 = 0; c0 < nb; c0 += kScanBlock) {
+    const int64_t b = c0 + threadIdx.x;
+    const int64_t x = b < nb ? adm_total(list[b]) : 0, inc = wave_incl_scan<int64_t>(x);
     __syncthreads();
-    int64_t bnx = run[kNumCls], bx = run[kNumCls + 1];
-    for (int v = 0; v < w; ++v) {
-      bnx += wsum[v][0];
-      bx += wsum[v][1];
-    }
-    const int64_t q_nx = bnx + __builtin_popcountll(m_nx & lanemask_lt());
-    const int64_t q_x = bx + __builtin_popcountll(m_x & lanemask_lt());
-    const bool drop = adm && (nx ? q_nx >= T : A0 + q_x >= T);
-    int k = valid ? (int)o.cls[i] : -1;
-    if (drop) {
-      k = (f & ELR_PLAN_N) ? ((f & ELR_PLAN_APP) ? kNApp : kNCmp)
-          : (f & ELR_PLAN_L) ? ((f & ELR_PLAN_APP) ? kLApp : kLCmp)
-          : (p.want_t ? kFNAdm : kS);
-      o.cls[i] = (int8_t)k;
-    }
-    const uint64_t m_cd = __builtin_amdgcn_ballot_w64(drop && nx);
-    const int rk = k >= 0 ? kRankOf[k] : -1;
-#pragma unroll
-    for (int q = 0; q < kNumCls; ++q) {
-      const uint64_t mq = __builtin_amdgcn_ballot_w64(rk == q);
-      if (lane == 0) wcls[w][q] = __builtin_popcountll(mq);
-    }
-    if (lane == 0) wsum[w][2] = __builtin_popcountll(m_cd);
+    if (lane == 63) wsum[w] = inc;
     __syncthreads();
-    if (threadIdx.x < kNumCls) {
-      const int q = threadIdx.x;
-      for (int sb = 0; sb < kScanBlock / kPlanBlock; ++sb) {
-        const int64_t blk = c0 / kPlanBlock + sb;
-        if (blk < nbu) bu2[(int64_t)q * nbu + blk] = run[q];
-        for (int v = sb * (kPlanBlock / 64); v < (sb + 1) * (kPlanBlock / 64); ++v) run[q] += wcls[v][q];
-      }
-    } else if (threadIdx.x < kNumCls + 3) {
-      const int q = threadIdx.x - kNumCls;
-      int64_t add = 0;
-      for (int v = 0; v < kRW; ++v) add += wsum[v][q];
-      run[threadIdx.x] += add;
+    int64_t before = run;
+    for (int v = 0; v < kRW; ++v) {
+      before += v < w ? wsum[v] : 0;
+      run += wsum[v];
     }
-    __syncthreads();
+    before += inc - x;
+    if (rank >= before && rank < before + x) {   // one block at most
+      cut_blk = b;
+      cut_rank = rank - before;
+    }
   }
-  if (threadIdx.x < kNumCls) tot2[threadIdx.x] = run[threadIdx.x];
   __syncthreads();
-  return run[kNumCls + 2];
+  // the cut's row, and its block's dropped rows by target
+  const int64_t cb = cut_blk, i = cb * kPlanBlock + threadIdx.x;
+  const int f = cb < nb && threadIdx.x < kPlanBlock && i < n ? o.flags[i] : 0;
+  const bool member = (f & ELR_PLAN_ADMIT) && ((f & ELR_PLAN_NEXT) != 0) == all;
+  const uint64_t m = __builtin_amdgcn_ballot_w64(member);
+  if (lane == 0 && w < kPlanBlock / 64) wcnt[w] = __builtin_popcountll(m);
+  __syncthreads();
+  if (member) {
+    int q = __builtin_popcountll(m & lanemask_lt());
+    for (int v = 0; v < w; ++v) q += wcnt[v];
+    if (q == (int)cut_rank) cut_row = i;
+  }
+  __syncthreads();
+  const DropCut cut{all ? 1 : 0, cut_row};
+  if (dropped(cut, f, i)) atomicAdd(&cut_pack, 1ull << (kAdmBits * drop_target(f)));
+  if (threadIdx.x == 0) *out_cut = cut;
+  __syncthreads();
+  // a wave per class: its offsets and total plus the rows dropped into it, or less those dropped from it
+  if (w < kNumCls) {
+    const int c = kClsOfRank[w];
+    const int fcls = p.want_t ? kFNAdm : kS;
+    // targets whose counts this class takes or gives up, as a mask, and the sign
+    const int mask = c == kNApp ? 1 : c == kNCmp ? 2 : c == kLApp ? 4 : c == kLCmp ? 8 : c == fcls ? 16
+                     : c == kNAdm ? 3 : c == kLAdm ? 12 : c == kFAdm ? 16 : 0;
+    const int sign = c == kNAdm || c == kLAdm || c == kFAdm ? -1 : 1;
+    int64_t carry = 0;
+    for (int64_t b0 = 0; b0 < nb; b0 += 64) {
+      const int64_t b = b0 + lane;
+      int x = 0;
+      if (b < nb) {
+        // this block's dropped rows: of the cut's list all past the cut's block, of the other list all or none
+        const int64_t past = b > cb ? list[b] : b == cb ? (int64_t)cut_pack : 0;
+        const int64_t rest = all && b != cb ? badm[nbu + b] : 0;   // (the cut's block: counted in cut_pack)
+#pragma unroll
+        for (int t = 0; t < kDropTargets; ++t)
+          if ((mask >> t) & 1) x += adm_field(past, t) + adm_field(rest, t);
+      }
+      const int inc = wave_incl_scan<int>(x);
+      if (b < nb) bu2[(int64_t)w * nbu + b] = bu[(int64_t)w * nbu + b] + sign * (carry + inc - x);
+      carry += __shfl(inc, 63, 64);
+    }
+    if (lane == 0) tot2[w] = tot[w] + sign * carry;
+  }
+  __syncthreads();
+  return all ? A0 - T : 0;
 }
 
 // The resolution of one step by the last block of the scan launch: everything the host planner decides from the
@@ -296,8 +360,8 @@ __device__ int64_t plan_overflow(const elr_plan_in& p, const elr_plan_out& o, in
 // into the step descriptor, with the dynamic pool's counters and the statistics advanced in the control state.
 // One thread decides; it loads everything it reads at once (a single round trip) and the stores go out together.
 __device__ void plan_resolve(const elr_plan_in& p, const elr_plan_out& o, const elr_plan_ctl& c, int64_t nbu,
-                             const int64_t* __restrict__ tot, int64_t* __restrict__ bu2,
-                             int64_t* __restrict__ tot2) {
+                             const int64_t* tot, const int64_t* bu, const int64_t* badm, int64_t* bu2, int64_t* tot2,
+                             DropCut* cut) {
   __shared__ int64_t sh[4];
   int64_t* S = c.state;
   int64_t* Dd = c.desc;
@@ -325,7 +389,7 @@ __device__ void plan_resolve(const elr_plan_in& p, const elr_plan_out& o, const 
   }
   __syncthreads();
   const int64_t need = sh[0];
-  const int64_t carry_drop = need > 0 ? plan_overflow(p, o, n, nbu, sh[2], need, bu2, tot2) : 0;
+  const int64_t carry_drop = need > 0 ? plan_overflow(p, o, n, nbu, sh[2], need, bu, tot, badm, bu2, tot2, cut) : 0;
   if (threadIdx.x != 0) return;
   const int64_t take = sh[1];
   if (need > 0) {   // the reclassified totals (the dynamic-slot ones stay), for the scatter launch too
@@ -438,7 +502,9 @@ __global__ __launch_bounds__(kScanBlock) void k_plan_scan_dev(elr_plan_in p, elr
                                                               int64_t nbd, int64_t* __restrict__ bu,
                                                               int64_t* __restrict__ bd, int64_t* __restrict__ bbad,
                                                               int64_t* __restrict__ tot, elr_plan_ctl ctl,
-                                                              int64_t* __restrict__ bu2, int64_t* __restrict__ tot2) {
+                                                              const int64_t* __restrict__ badm,
+                                                              int64_t* __restrict__ bu2, int64_t* __restrict__ tot2,
+                                                              DropCut* __restrict__ cut) {
   __shared__ int64_t stot[kPlanCh];
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
   if (c < kPlanCh) {
@@ -471,7 +537,7 @@ __global__ __launch_bounds__(kScanBlock) void k_plan_scan_dev(elr_plan_in p, elr
     }
   }
   __syncthreads();
-  plan_resolve(p, o, ctl, nbu, stot, bu2, tot2);
+  plan_resolve(p, o, ctl, nbu, stot, bu, badm, bu2, tot2, cut);
 }
 
 // Pass 3: stable scatter by class.
@@ -481,15 +547,27 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_scatter(elr_plan_in p, elr_
                                                              const int64_t* __restrict__ tot_in,
                                                              const int64_t* __restrict__ desc,
                                                              const int64_t* __restrict__ bu2,
-                                                             const int64_t* __restrict__ tot2) {
+                                                             const int64_t* __restrict__ tot2,
+                                                             const DropCut* __restrict__ cut) {
   const int64_t b = blockIdx.x;
-  // after the device-driven overflow path: its reclassified offsets and totals
+  // after the device-driven overflow path: its reclassified offsets and totals, the rows past its cut reclassified
   const bool ovf = desc && desc[kDOverflow] > 0;
   const int64_t* __restrict__ bu = ovf ? bu2 : bu_in;
   const int64_t* __restrict__ tot = ovf ? tot2 : tot_in;
   if (b < nbu) {
     const int64_t i = b * kPlanBlock + threadIdx.x;
-    const int k = i < rows_n(p) ? kRankOf[(int)o.cls[i]] : -1;
+    int k = -1;
+    if (i < rows_n(p)) {
+      int cls = o.cls[i];
+      if (ovf) {
+        const int f = o.flags[i];
+        if (dropped(*cut, f, i)) {
+          cls = drop_class(f, p.want_t);
+          o.cls[i] = (int8_t)cls;
+        }
+      }
+      k = kRankOf[cls];
+    }
     int t[kNumCls];
     const int r = block_class_rank<kNumCls>(k, t);
     if (k >= 0) {
@@ -594,20 +672,25 @@ static int plan_classify_launch(const elr_plan_in& p, const elr_plan_out& o, voi
   elr_plan_ctl c{};
   int64_t* bu2 = nullptr;
   int64_t* tot2 = nullptr;
+  int64_t* badm = nullptr;
+  DropCut* cut = nullptr;
   if (ctl) {
     c = *ctl;
     bu2 = (int64_t*)((char*)scratch + elr_plan_scratch_bytes(p.n, p.nd));
     tot2 = bu2 + kNumCls * nbu;
+    cut = (DropCut*)(tot2 + 16);
+    badm = tot2 + 18;
   }
-  const PlanCount count{p, o, nbu, nbd, bu, bd, bbad};
+  const PlanCount count{p, o, nbu, nbd, bu, bd, bbad, badm};
   if (seg && seg->blocks > 0)
     seg_partials_visit(*seg, [&](const auto& f, int64_t nb) { launch2(count, nbu + nbd, f, nb, st); });
   else
     launch1(count, nbu + nbd, st);
-  if (ctl) k_plan_scan_dev<<<1, kScanBlock, 0, st>>>(p, o, nbu, nbd, bu, bd, bbad, tot, c, bu2, tot2);
+  if (ctl) k_plan_scan_dev<<<1, kScanBlock, 0, st>>>(p, o, nbu, nbd, bu, bd, bbad, tot, c, badm, bu2, tot2, cut);
   else k_plan_scan<<<kPlanCh, kScanBlock, 0, st>>>(p, o, nbu, nbd, bu, bd, bbad, tot);
   if (nbu + nbd > 0)
-    k_plan_scatter<<<(unsigned)(nbu + nbd), kPlanBlock, 0, st>>>(p, o, nbu, nbd, bu, bd, tot, c.desc, bu2, tot2);
+    k_plan_scatter<<<(unsigned)(nbu + nbd), kPlanBlock, 0, st>>>(p, o, nbu, nbd, bu, bd, tot, c.desc, bu2, tot2,
+                                                                      cut);
   return launch_status();
 }
 
@@ -636,7 +719,8 @@ extern "C" int64_t elr_plan_step_scratch_bytes(int64_t n, int64_t nd) {
   using namespace elr;
   const int64_t base = elr_plan_scratch_bytes(n, nd);
   if (base < 0) return base;
-  return base + (((kNumCls * plan_blocks(n) + 16) * 8 + 255) & ~int64_t(255));
+  // bu2, tot2 and the cut of the overflow path, the blocks' counts of admitted rows
+  return base + ((((kNumCls + 2) * plan_blocks(n) + 18) * 8 + 255) & ~int64_t(255));
 }
 
 extern "C" int elr_plan_step(const elr_plan_in* in, const elr_plan_out* out, const elr_plan_ctl* ctl, void* scratch,

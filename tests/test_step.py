@@ -602,3 +602,89 @@ def test_gpu_plan_admit_slots_matches_stack_arithmetic(dev, n_free, nev, n_adm, 
     assert (dyn.cpu().numpy()[nkeep + n_adm:] == -7).all()
     for x, y in zip(o, g):
         assert torch.equal(x, y.cpu())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,carry,want_t,drop', [
+    (1, False, True, 'all'), (256, False, True, 'few'), (257, True, False, 'to_next'), (5_000, True, True, 'into_next'),
+    (70_001, False, False, 'few'), (300_003, True, True, 'few'), (300_003, False, True, 'into_next'),
+    (300_003, False, False, 'all')])
+def test_gpu_plan_step_overflow_cut(dev, n, carry, want_t, drop):
+    """elr_plan_step with more admissions than free slots, against a numpy restatement of srm2/elara.py:246-258: the
+    dropped admissions (few: rows outside the next batches; to_next: all of those; into_next: also rows of the next
+    batches; all), the classes, the class order and the counts.  Up to 1,172 blocks of rows, past the resolving block's
+    1,024 threads."""
+    import ctypes
+    from elara_amd import _lib
+    print(f'[gpu-test] plan step overflow n={n} carry={carry} want_t={want_t} drop={drop}', flush=True)
+    rng = np.random.default_rng(n + 7 * carry)
+    R, K, s = 2 * n + 5, 3, 9
+    u = np.sort(rng.choice(R, n, replace=False)).astype(np.int64)
+    slot_of = np.where(rng.random(R) < 0.3, 0, -1).astype(np.int32)
+    seen = rng.integers(s - 2, s + 5, R).astype(np.int32)
+    code = rng.choice(np.array([0, 0, 1, 2, 3, K + 1], np.int8), R)
+    bits = rng.integers(0, 16, R).astype(np.int32) << (s + 1)     # steps s+1 .. s+4 of the ring
+    mask = 3 << (s + 1)
+    if n == 1:
+        slot_of[:], seen[:] = -1, s + 1
+        bits[:] = mask
+    toff, kthr = np.array([0, R // 2], np.int64), np.array([1, 3], np.int8)
+    # the classes before any drop
+    sl, c, nx = slot_of[u], code[u].astype(int), (bits[u] & mask) != 0
+    adm = (sl < 0) & (nx if carry else seen[u] > s)
+    app = c < kthr[(u >= toff[1]).astype(int)]
+    n_adm, a0 = int(adm.sum()), int((adm & nx).sum())
+    need = {'all': n_adm, 'few': max(1, (n_adm - a0) // 3), 'to_next': n_adm - a0, 'into_next': n_adm - a0 // 2}[drop]
+    need = min(max(need, 1), n_adm)
+
+    def classes(a):
+        N, L = c == 0, (c >= 1) & (c <= K)
+        return np.where(sl >= 0, 0, np.where(N, np.where(a, 1, np.where(app, 2, 3)),
+                        np.where(L, np.where(a, 4, np.where(app, 5, 6)),
+                                 np.where(a, 7, 8 if want_t else 9))))
+    pri = np.where(adm, np.where(nx, 0, 2), 4)
+    kept = adm.copy()
+    kept[np.argsort(pri, kind='stable')[n_adm - need:n_adm]] = False
+    cls = classes(kept)
+    rank_of = np.array([0, 1, 4, 6, 2, 5, 7, 3, 8, 9])
+    order = np.argsort(rank_of[cls], kind='stable')
+    tot = np.bincount(rank_of[cls], minlength=10)
+
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    e = lambda m, dt: torch.full((max(m, 1),), -7, dtype=dt, device=dev)  # noqa: E731
+    I8, I32, I64, U8 = torch.int8, torch.int32, torch.int64, torch.uint8
+    keep = dict(u=t(u), slot_of=t(slot_of), last_seen=t(seen), code=t(code), kthr=t(kthr), toff=t(toff), next_bits=t(bits),
+                loc=t(np.arange(R + 1, dtype=np.int32)), slot_row=t(np.full(4, -1, np.int64)), dyn=e(4, I64),
+                tops=torch.zeros(3, dtype=I64, device=dev), nd=torch.zeros(1, dtype=I64, device=dev))
+    out = dict(cls=e(n, I8), flags=e(n, U8), sl=e(n, I32), c=e(n, I8), order=e(n, I64), rank=e(n, I64), dyn_out=e(8, I64),
+               counts=e(17, I64), u_ord=e(n, I64), c_ord=e(n, I64), sl_ord=e(n, I64), L_row=e(n, I64), L_cnt=e(n, I32),
+               loc_ord=e(n, I64))
+    state = torch.zeros(_lib.CTL_WORDS, dtype=I64, device=dev)
+    state[_lib.S_NFREE] = n_adm - need
+    desc = torch.zeros(_lib.DESC_WORDS, dtype=I64, device=dev)
+    p, o, ctl = _lib.PlanIn(), _lib.PlanOut(), _lib.PlanCtl()
+    for f in ('u', 'slot_of', 'last_seen', 'code', 'kthr', 'toff', 'next_bits', 'loc', 'slot_row', 'dyn'):
+        setattr(p, f, keep[f].data_ptr())
+    p.n, p.T, p.nd, p.s, p.K, p.want_t, p.R, p.next_mask, p.carry = n, 2, 4, s, K, int(want_t), R, mask, int(carry)
+    p.mat_top, p.log_top, p.live = (keep['tops'][i:].data_ptr() for i in range(3))
+    p.nd_dev = keep['nd'].data_ptr()
+    for f, x in out.items():
+        setattr(o, f, x.data_ptr())
+    ctl.state, ctl.desc, ctl.mat_cap, ctl.log_cap = state.data_ptr(), desc.data_ptr(), 10 * n, 10 * n
+    L = _lib.lib()
+    nb = int(L.elr_plan_step_scratch_bytes(n, 4))
+    scratch = torch.empty(nb, dtype=U8, device=dev)
+    rc = L.elr_plan_step(ctypes.byref(p), ctypes.byref(o), ctypes.byref(ctl), scratch.data_ptr(), nb, None, 0, 64, 20,
+                         None, 0, torch.cuda.current_stream(dev).cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    d = desc.tolist()
+    assert d[_lib.D_SKIP] == 0 and d[_lib.D_OVERFLOW] == need
+    assert d[_lib.D_BARRIER] == int((adm & nx & ~kept).any())
+    assert d[_lib.D_B:_lib.D_B + 11] == [0, *np.cumsum(tot).tolist()]
+    assert np.array_equal(out['cls'][:n].cpu().numpy(), cls)
+    assert np.array_equal(out['order'][:n].cpu().numpy(), order)
+    assert np.array_equal(out['u_ord'][:n].cpu().numpy(), u[order])
+    assert np.array_equal(out['rank'][:n].cpu().numpy()[order], np.arange(n))
+    Ls = np.concatenate([u[cls == k] for k in (4, 5, 6)])
+    assert np.array_equal(out['L_row'][:Ls.size].cpu().numpy(), Ls)
