@@ -6,16 +6,16 @@
 // segment sum, Adam on each unique row).
 //
 // Sort.  Stable LSD radix sort of (id, occurrence index) pairs, 8-bit digits, ceil(key_bits / 8) passes (or one
-// pass fewer with 9- or 10-bit digits), keys held as uint32 when key_bits <= 32.  Tiles of 4096 keys, or 1024 below
-// 2^18 keys.  A pass is three launches: per-tile digit histograms, a wave per digit scanning that digit's per-tile
+// pass fewer with 9- or 10-bit digits), keys held as uint32 when key_bits <= 32, in tiles of 4096 keys.  A pass is
+// per-tile digit histograms, above kSortFoldTiles tiles a launch of a wave per digit scanning that digit's per-tile
 // counts, and a scatter in which each key's rank among equal digits of its tile comes from wave ballots (peer mask
 // of the digit bits), a per-wave running count in LDS and a scan over the tile's waves, so equal keys keep their
 // occurrence order.
 //
 // Segments.  Sorted position i starts a segment when its key differs from position i-1; per-block head counts, then
 // a launch in which each block adds up the counts of the blocks before it (or, above kFoldMaxBlocks blocks, a
-// one-block scan launch in between), gives every position its unique index (the inverse) and every unique id its
-// first position.  The extra-chunk plan is laid out the same way.
+// one-block scan launch in between), gives every position its unique index (the inverse), every unique id its
+// first position, and lays out the partial chunks of the long segments.
 //
 // Summation order: ATen's, as torch.ops.aten.embedding_dense_backward computes it on this GPU
 // (aten/src/ATen/native/cuda/Embedding.cu embedding_dense_backward_cuda and EmbeddingBackwardKernel.cu, PyTorch
@@ -35,27 +35,32 @@
 
 namespace elr {
 
-constexpr int kSortThreads = 256;
-// Keys per thread of a sort tile and positions per thread of a segment tile: 16 (tiles of 4,096) from kBigBatch
-// keys, 4 below it, so that a small batch still spreads over a few hundred blocks.  The threshold is set for a batch
-// sorted beside other kernels, as the ELARA step sorts the batches it loads ahead: at config C5 (425,984 keys)
-// tiles of 4,096 make a sort alone 124 us against 81 us with tiles of 1,024, but its launches of a quarter as many
-// blocks take fewer CUs from the step's kernels beside them, and the step is faster (0.342 against 0.357 ms
-// device-driven, 0.279 against 0.297 ms host-planned; three alternations on one box; tiles of 2,048 in between,
-// 8,192 slower than both).
-constexpr int kItemsBig = 16;
-constexpr int kItemsSmall = 4;
-constexpr int64_t kBigBatch = int64_t(1) << 18;
-inline int items_for(int64_t n) { return n >= kBigBatch ? kItemsBig : kItemsSmall; }
-constexpr int kRadixBins = 256;      // bins of an 8-bit digit; passes take 8, 9 or 10 bits (sort_plan)
-constexpr int kRadixMaxBits = 10;
+// A sort tile is 4,096 keys: 1,024 threads with 4 keys each below kSortBig keys, where a tile's chain of ranking rounds
+// and LDS passes is what a launch takes (the scatters of 426k keys 9 us against 13.5 with 256 threads of 16 keys), and
+// 256 threads with 16 keys each from there, where several tiles per CU hide it (3.4M keys: 26 us against 36).
+constexpr int kSortTile = 4096;
+constexpr int kSortThreadsSmall = 1024;
+constexpr int kSortThreadsBig = 256;
+constexpr int64_t kSortBig = int64_t(1) << 20;
+inline int64_t sort_tiles(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
+// Up to this many tiles every scatter block adds up the tiles' digit counts itself; above, a launch of a wave per digit
+// scans them (k_radix_hist_scan).  At 104 tiles the scans' launches (4.2 us each) cost more than the sums: a batch of
+// 426k ids sorted twice 312 against 303 us, and at 26 tiles 99 against 92 us for the whole duplicate-id update.
+constexpr int64_t kSortFoldTiles = 128;
+static_assert(kSortFoldTiles * kSortTile <= kSortBig, "the scatters that sum the counts have 1,024 threads");
+// Rounds of a segment tile (k_seg_count, k_seg_apply): 8 from 2^20 positions, 4 below, so that a small batch still
+// spreads over the chip (426k positions: 8 us against 19 with 16 rounds; 3.4M: 27 us with 8 rounds, 29 with 16).
+constexpr int kSegItemsBig = 8;
+constexpr int kSegItemsSmall = 4;
+constexpr int64_t kSegBig = int64_t(1) << 20;
+inline int seg_items_for(int64_t n) { return n >= kSegBig ? kSegItemsBig : kSegItemsSmall; }
+constexpr int kRadixMaxBits = 10;   // passes take digits of 8, 9 or 10 bits (sort_plan)
 constexpr int kRadixMaxBins = 1 << kRadixMaxBits;
 constexpr int64_t kAtenSmall = 3072;                      // ATen's windowed path up to this many indices
 constexpr int kAtenWinShift = 4;                          // its window: 16 indices
+constexpr int64_t kWinHot = 64;                           // windowed segments longer than this are hot (SegFinalSub)
 constexpr int kSegParts = 8;                              // run sums a final-kernel wave loads together
 constexpr int kSegBlock = 256;
-
-static_assert(kSortThreads == kRadixBins, "at least one histogram bin per sort thread");
 
 template <int RB, typename Key>
 __device__ __forceinline__ uint32_t digit_of(Key k, int shift) {
@@ -78,53 +83,45 @@ inline void sort_plan(int key_bits, int max_bits, int& passes, int& rb) {
   rb = 8;
 }
 
-// Per-tile histogram of RB-bit digits, digit-major: hist[d * nblk + tile].
-template <typename Src, typename Key, int ITEMS, int RB>
-__global__ __launch_bounds__(kSortThreads) void k_radix_hist(const Src* __restrict__ src, int64_t n, int shift,
-                                                             int64_t* __restrict__ hist, int64_t nblk) {
-  constexpr int BINS = 1 << RB;
+// Per-tile histogram of RB-bit digits: digit-major (hist[d * ntile + tile]) for k_radix_hist_scan, tile-major
+// (hist[tile * BINS + d]) when the scatter adds the counts up itself (fold).
+template <typename Src, typename Key, int RB, int NT>
+__global__ __launch_bounds__(NT) void k_radix_hist(const Src* __restrict__ src, int64_t n, int shift,
+                                                   int32_t* __restrict__ hist, int64_t ntile, int fold) {
+  constexpr int BINS = 1 << RB, ITEMS = kSortTile / NT;
   __shared__ int h[BINS];
-  for (int b = threadIdx.x; b < BINS; b += kSortThreads) h[b] = 0;
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kSortThreads * ITEMS;
+  const int t = threadIdx.x;
+  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+  Key kk[ITEMS];
+#pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
-    const int64_t pos = base + (int64_t)r * kSortThreads + threadIdx.x;
-    if (pos < n) atomicAdd(&h[digit_of<RB>((Key)src[pos], shift)], 1);
+    const int64_t pos = base + r * NT + t;
+    kk[r] = pos < n ? (Key)src[pos] : (Key)0;
   }
+  for (int b = t; b < BINS; b += NT) h[b] = 0;
   __syncthreads();
-  for (int b = threadIdx.x; b < BINS; b += kSortThreads) hist[(int64_t)b * nblk + blockIdx.x] = h[b];
-}
-
-// Exclusive prefix over BINS values held BPT per thread (thread t holds bins t*BPT .. t*BPT + BPT - 1, in x[]):
-// the prefixes to ex[], the total of all bins to *total.
-template <int BPT>
-__device__ __forceinline__ void bins_excl_scan(const int (&x)[BPT], int (&ex)[BPT], int& total) {
-  int loc = 0;
 #pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    ex[j] = loc;
-    loc += x[j];
-  }
-  int v[1] = {loc}, e[1], tot[1];
-  block_excl_scan<kSortThreads, 1>(v, e, tot);
-#pragma unroll
-  for (int j = 0; j < BPT; ++j) ex[j] += e[0];
-  total = tot[0];
+  for (int r = 0; r < ITEMS; ++r)
+    if (base + r * NT + t < n) atomicAdd(&h[digit_of<RB>(kk[r], shift)], 1);
+  __syncthreads();
+  for (int b = t; b < BINS; b += NT)
+    hist[fold ? (int64_t)blockIdx.x * BINS + b : (int64_t)b * ntile + blockIdx.x] = h[b];
 }
 
 // One wave per digit: exclusive scan of that digit's per-tile counts (in place) and the digit's total.  The wave
 // loads up to 512 counts (8 per lane) before it scans them, so a few hundred tiles cost one round of loads; no
 // block barrier.
-__global__ __launch_bounds__(kSortThreads) void k_radix_hist_scan(int64_t* __restrict__ hist, int64_t ntile,
-                                                                  int nbins, int64_t* __restrict__ dtot) {
-  constexpr int kWaves = kSortThreads / 64, kPer = 8;
+constexpr int kHistScanThreads = 256;
+__global__ __launch_bounds__(kHistScanThreads) void k_radix_hist_scan(int32_t* __restrict__ hist, int64_t ntile,
+                                                                      int nbins, int32_t* __restrict__ dtot) {
+  constexpr int kWaves = kHistScanThreads / 64, kPer = 8;
   const int lane = threadIdx.x & 63;
   const int d = blockIdx.x * kWaves + (threadIdx.x >> 6);
   if (d >= nbins) return;
-  int64_t* h = hist + (int64_t)d * ntile;
-  int64_t carry = 0;
+  int32_t* h = hist + (int64_t)d * ntile;
+  int carry = 0;   // n < 2^31
   for (int64_t g0 = 0; g0 < ntile; g0 += 64 * kPer) {
-    int64_t x[kPer];
+    int x[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const int64_t b = g0 + k * 64 + lane;
@@ -133,7 +130,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_hist_scan(int64_t* __res
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const int64_t b = g0 + k * 64 + lane;
-      const int64_t inc = wave_incl_scan<int64_t>(x[k]);
+      const int inc = wave_incl_scan<int>(x[k]);
       if (b < ntile) h[b] = carry + inc - x[k];
       carry += __shfl(inc, 63, 64);
     }
@@ -146,29 +143,56 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_blocks(int64_t* __restrict_
   scan_channels_block(bsum, n, 1, nullptr);
 }
 
+// The lanes of this wave (of those for which valid holds) whose RB-bit digit d equals this lane's.
+__device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid, int rb) {
+  uint64_t m = __ballot(valid);
+#pragma unroll
+  for (int b = 0; b < rb; ++b) {
+    const bool bit = (d >> b) & 1u;
+    const uint64_t bal = __ballot(bit);
+    m &= bit ? bal : ~bal;
+  }
+  return m;
+}
+
+// Exclusive prefix over values held BPT per thread of an NT-thread block (in thread order): put(j, prefix of x[j]).
+template <int NT, int BPT, class Put>
+__device__ __forceinline__ void bins_excl_scan(const int (&x)[BPT], Put&& put) {
+  int v[1] = {0}, e[1], tot[1];
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) v[0] += x[j];
+  block_excl_scan<NT, 1>(v, e, tot);
+#pragma unroll
+  for (int j = 0; j < BPT; ++j) {
+    put(j, e[0]);
+    e[0] += x[j];
+  }
+}
+
 // Stable scatter of one pass.  FIRST: the source keys are the caller's int64 ids and the values are their
-// positions.  Wave w of the block takes the tile's w-th quarter, 64 consecutive positions per round, so an item's
-// rank among the tile's items of its digit is: items of that digit in earlier waves' quarters, plus those of its
+// positions.  Wave w of the block takes the tile's w-th part, 64 consecutive positions per round, so an item's
+// rank among the tile's items of its digit is: items of that digit in earlier waves' parts, plus those of its
 // own wave's earlier rounds (a per-wave running count in LDS, which only that wave touches, in program order), plus
 // its peers in the same round below its lane (ballots).  The waves run their rounds without block barriers; one
 // scan over the waves' counts per digit at the end gives the first term.  The tile is then sorted by digit in LDS
 // and written out run by run, so consecutive threads write consecutive addresses of one digit's bucket instead of
-// 64 scattered ones.
-template <typename Src, typename Key, bool FIRST, int ITEMS, int RB>
-__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const Src* __restrict__ src_keys,
+// 64 scattered ones.  A digit's first position for this tile: the exclusive scan of the digit totals plus the
+// earlier tiles' counts, both from the scan launch (offs, dtot) or, with fold, summed here from the tile-major
+// histograms.
+template <typename Src, typename Key, bool FIRST, int RB, int NT>
+__global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ src_keys,
                                                                 const int32_t* __restrict__ src_vals, int64_t n,
-                                                                int shift, const int64_t* __restrict__ offs,
-                                                                const int64_t* __restrict__ dtot, int64_t nblk,
+                                                                int shift, const int32_t* __restrict__ offs,
+                                                                const int32_t* __restrict__ dtot, int ntile, int fold,
                                                                 Key* __restrict__ dst_keys,
                                                                 int32_t* __restrict__ dst_vals) {
-  constexpr int NW = kSortThreads / 64;
-  constexpr int TILE = kSortThreads * ITEMS;
-  constexpr int BINS = 1 << RB, BPT = BINS / kSortThreads;   // digits per thread in the per-digit steps
-  static_assert(BPT * kSortThreads == BINS, "RB >= 8");
-  __shared__ int bo[BINS];       // global position of this tile's first item of digit d (n < 2^31)
-  __shared__ int run[BINS];      // items of digit d in the tile
-  __shared__ int lbase[BINS];    // position of digit d's first item in the tile sorted by digit
-  __shared__ int wc[NW][BINS];   // per wave: running count of digit d, then the count in earlier waves
+  constexpr int TILE = kSortTile, ITEMS = TILE / NT, NW = NT / 64;
+  constexpr int BINS = 1 << RB;
+  constexpr int G = NT > BINS ? NT / BINS : 1;      // groups of threads that share the tiles' counts (fold)
+  constexpr int BPT = BINS > NT ? BINS / NT : 1;    // digits per thread, digit t * BPT + j
+  __shared__ int bo[BINS];            // global position of this tile's first item of digit d (n < 2^31)
+  __shared__ int lbase[BINS];         // position of digit d's first item in the tile sorted by digit
+  __shared__ uint16_t wc[NW][BINS];   // per wave: running count of digit d, then the count in earlier waves
   __shared__ Key lk[TILE];
   __shared__ int32_t lv[TILE];
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
@@ -183,72 +207,81 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const Src* __res
     kk[r] = valid ? (Key)src_keys[pos] : (Key)0;
     vv[r] = valid ? (FIRST ? (int32_t)pos : src_vals[pos]) : 0;
   }
-  {
-    // digit bases: exclusive scan of the digit totals (n < 2^31, so they fit in int)
-    int x[BPT], ex[BPT], total;
+  const bool own = t * BPT < BINS;   // this thread's digits
+  int first[BPT], total[BPT];        // their items in earlier tiles and in all tiles
 #pragma unroll
-    for (int j = 0; j < BPT; ++j) x[j] = (int)dtot[t * BPT + j];
-    bins_excl_scan<BPT>(x, ex, total);
+  for (int j = 0; j < BPT; ++j) first[j] = total[j] = 0;
+  if (NT == kSortThreadsSmall && fold) {
+    const int d = t & (BINS - 1), g = t / BINS;
+    int* part = lv;   // 2 * NT ints
+    static_assert(NT != kSortThreadsSmall || (2 * NT <= TILE && BPT == 1), "the groups' sums fit in the tile's LDS");
+    int x0 = 0, x1 = 0;
+#pragma unroll 8
+    for (int b = g; b < ntile; b += G) {
+      const int x = offs[b * BINS + d];
+      x0 += b < (int)blockIdx.x ? x : 0;
+      x1 += x;
+    }
+    part[t] = x0;
+    part[NT + t] = x1;
+    __syncthreads();
+    if (own)
 #pragma unroll
-    for (int j = 0; j < BPT; ++j) bo[t * BPT + j] = ex[j] + (int)offs[(int64_t)(t * BPT + j) * nblk + blockIdx.x];
+      for (int q = 0; q < G; ++q) {
+        first[0] += part[q * BINS + t];
+        total[0] += part[NT + q * BINS + t];
+      }
+  } else if (own) {
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+      first[j] = offs[(int64_t)(t * BPT + j) * ntile + blockIdx.x];
+      total[j] = dtot[t * BPT + j];
+    }
   }
-#pragma unroll
-  for (int q = 0; q < NW; ++q)
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) wc[q][t * BPT + j] = 0;
+  bins_excl_scan<NT, BPT>(total, [&](int j, int ex) {
+    if (own) bo[t * BPT + j] = ex + first[j];
+  });
+  for (int q = t; q < NW * BINS / 2; q += NT) reinterpret_cast<uint32_t*>(&wc[0][0])[q] = 0;
   __syncthreads();
   int rk[ITEMS];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
-    const int64_t pos = base + (int64_t)r * 64 + lane;
-    const bool valid = pos < n;
+    const bool valid = base + (int64_t)r * 64 + lane < n;
     const uint32_t d = digit_of<RB>(kk[r], shift);
-    uint64_t m = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bal = __ballot(bit);
-      m &= bit ? bal : ~bal;
-    }
+    const uint64_t m = digit_peers(d, valid, RB);
     const int lr = __popcll(m & lanemask_lt());
     // every lane reads its digit's running count before the group's lowest lane adds the group's size: one wave's
     // LDS accesses take effect in program order
-    const int before = valid ? wc[w][d] : 0;
+    const int before = valid ? (int)wc[w][d] : 0;
     rk[r] = valid ? before + lr : -1;
-    if (valid && lr == 0) wc[w][d] = before + __popcll(m);
+    if (valid && lr == 0) wc[w][d] = (uint16_t)(before + __popcll(m));
   }
   __syncthreads();
-  int runs[BPT];
-#pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    // per digit: exclusive scan over the waves, and the tile's total
-    const int dd = t * BPT + j;
-    int acc = 0;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) {
-      const int c = wc[q][dd];
-      wc[q][dd] = acc;
-      acc += c;
-    }
-    runs[j] = acc;
-    run[dd] = acc;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < ITEMS; ++r)
-    if (rk[r] >= 0) rk[r] += wc[w][digit_of<RB>(kk[r], shift)];
   {
-    // the tile sorted by digit: digit d's items start at the exclusive scan of the tile's digit counts
-    int ex[BPT], total;
-    bins_excl_scan<BPT>(runs, ex, total);
+    // per digit: exclusive scan over the waves, then the tile sorted by digit: digit d's items start at the exclusive
+    // scan of the tile's digit counts
+    int x[BPT];
 #pragma unroll
-    for (int j = 0; j < BPT; ++j) lbase[t * BPT + j] = ex[j];
+    for (int j = 0; j < BPT; ++j) {
+      x[j] = 0;
+      if (own)
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+          const int c = wc[q][t * BPT + j];
+          wc[q][t * BPT + j] = (uint16_t)x[j];
+          x[j] += c;
+        }
+    }
+    bins_excl_scan<NT, BPT>(x, [&](int j, int ex) {
+      if (own) lbase[t * BPT + j] = ex;
+    });
   }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     if (rk[r] >= 0) {
-      const int lp = lbase[digit_of<RB>(kk[r], shift)] + rk[r];
+      const uint32_t d = digit_of<RB>(kk[r], shift);
+      const int lp = lbase[d] + wc[w][d] + rk[r];
       lk[lp] = kk[r];
       lv[lp] = vv[r];
     }
@@ -256,41 +289,97 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const Src* __res
   __syncthreads();
   const int64_t rem = n - tile0;
   const int nvalid = rem < TILE ? (int)rem : TILE;
-  for (int j = t; j < nvalid; j += kSortThreads) {
-    const Key k = lk[j];
-    const uint32_t d = digit_of<RB>(k, shift);
-    const int64_t dst = (int64_t)bo[d] + (j - lbase[d]);
-    if (dst >= 0 && dst < n) {
-      dst_keys[dst] = k;
-      dst_vals[dst] = lv[j];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = r * NT + t;
+    if (j < nvalid) {
+      const Key k = lk[j];
+      const uint32_t d = digit_of<RB>(k, shift);
+      const int64_t dst = (int64_t)bo[d] + (j - lbase[d]);
+      if (dst >= 0 && dst < n) {
+        dst_keys[dst] = k;
+        dst_vals[dst] = lv[j];
+      }
     }
   }
 }
 
-// Segment kernels take a tile of kSegBlock * ITEMS positions per block, in ITEMS rounds of kSegBlock consecutive
-// positions (thread t takes position base + r * kSegBlock + t in round r: every load is coalesced).  Positions are
-// ranked in that order, round by round, with one block scan per round.
+// Segment kernels take a tile of kSegBlock * ITEMS positions per block: wave w of the block the tile's w-th quarter,
+// ITEMS rounds of 64 consecutive positions.  A position starts a segment (is a head) when its key differs from the one
+// before it; a round's heads are one ballot, so positions are ranked with popcounts of the wave's ITEMS masks and the
+// block synchronises once, not once per round.
+constexpr int kSegWaves = kSegBlock / 64;
 
-template <typename Key>
-__device__ __forceinline__ int is_head(const Key* __restrict__ sk, int64_t i, int64_t n) {
-  return i < n && (i == 0 || sk[i] != sk[i - 1]) ? 1 : 0;
+// x of lane l, and the block's wave index, as wave-uniform (scalar) values.
+__device__ __forceinline__ int lane_value(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
+__device__ __forceinline__ int block_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// The wave's keys of sorted positions p0 + r * 64 + lane, and each round's head mask.
+template <typename Key, int ITEMS>
+__device__ __forceinline__ void seg_heads(const Key* __restrict__ sk, int64_t p0, int64_t n, Key (&kk)[ITEMS],
+                                          uint64_t (&hm)[ITEMS]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = p0 + r * 64 + lane;
+    kk[r] = i < n ? sk[i] : (Key)0;
+  }
+  Key prev = p0 > 0 && p0 < n ? sk[p0 - 1] : (Key)0;   // the key before the round
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = p0 + r * 64 + lane;
+    Key left = __shfl_up(kk[r], 1, 64);
+    if (lane == 0) left = prev;
+    hm[r] = __builtin_amdgcn_ballot_w64(i < n && (i == 0 || kk[r] != left));
+    prev = __shfl(kk[r], 63, 64);
+  }
 }
 
-// Segment heads: per-block head counts.
+// Segment heads: per-block head counts and first head position (n when the tile has none).  Also clears the counts
+// that k_seg_apply's chunk plan adds to.
 template <typename Key, int ITEMS>
 __global__ __launch_bounds__(kSegBlock) void k_seg_count(const Key* __restrict__ sk, int64_t n,
-                                                         int64_t* __restrict__ bsum) {
-  const int64_t base = (int64_t)blockIdx.x * kSegBlock * ITEMS + threadIdx.x;
-  int v[1] = {0}, ex[1], tot[1];
-  for (int r = 0; r < ITEMS; ++r) v[0] += is_head(sk, base + (int64_t)r * kSegBlock, n);
-  block_excl_scan<kSegBlock, 1>(v, ex, tot);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = tot[0];
+                                                         int64_t* __restrict__ bsum, int32_t* __restrict__ bfirst,
+                                                         int64_t* __restrict__ d_E, int64_t* __restrict__ d_hot) {
+  __shared__ int wcnt[kSegWaves];
+  __shared__ int wfirst[kSegWaves];
+  const int w = block_wave();
+  const int64_t p0 = ((int64_t)blockIdx.x * kSegWaves + w) * (64 * ITEMS);
+  Key kk[ITEMS];
+  uint64_t hm[ITEMS];
+  seg_heads<Key, ITEMS>(sk, p0, n, kk, hm);
+  int c = 0;
+  int first = (int)n;
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    c += __builtin_popcountll(hm[r]);
+    if (hm[r]) first = (int)p0 + r * 64 + __builtin_ctzll(hm[r]);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    wcnt[w] = c;
+    wfirst[w] = first;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    int f = (int)n;
+    for (int v = 0; v < kSegWaves; ++v) {
+      t += wcnt[v];
+      f = wfirst[v] < f ? wfirst[v] : f;
+    }
+    bsum[blockIdx.x] = t;
+    bfirst[blockIdx.x] = f;
+    if (blockIdx.x == 0) {
+      *d_E = 0;
+      *d_hot = 0;
+    }
+  }
 }
 
-// Grids of at most this many blocks take their block offsets by block_offset; larger ones from a one-block scan
-// launch (k_scan_blocks) between the count and apply launches.  At config C3 (830 blocks) the summing blocks made the
-// step 55 us slower where the sort runs beside the final segment kernel; at C5 (104 blocks) they save the launch.
-constexpr int64_t kFoldMaxBlocks = 256;
+// Grids of at most this many blocks take their block offsets by block_offset (a block reads at most 8 counts per
+// thread); larger ones from a one-block scan launch (k_scan_blocks) between the count and apply launches (4.5 us; at
+// config C3's 1,664 blocks the sums in the blocks save 3 us).
+constexpr int64_t kFoldMaxBlocks = 2048;
 
 // Sum of cnt[0 .. b) over the whole block, returned to every thread: the offset of block b from the per-block
 // counts of the launch before, without a scan launch in between.
@@ -305,46 +394,7 @@ __device__ __forceinline__ int64_t block_offset(const int64_t* __restrict__ cnt,
   int64_t t = 0;
 #pragma unroll
   for (int q = 0; q < kSegBlock / 64; ++q) t += wpart[q];
-  __syncthreads();   // wpart is reused by the caller's next call
   return t;
-}
-
-// Segment heads: unique ids, segment starts, each segment's first occurrence index and the inverse.  The block's
-// first segment index: the sum of the earlier blocks' head counts (k_seg_count), or, with `scanned`, bcnt[block]
-// after k_scan_blocks.  The last block stores U to d_U (and n_unique) and seg_start[U] = n.
-template <typename Key, int ITEMS>
-__global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__ sk, const int32_t* __restrict__ sv,
-                                                         int64_t n, const int64_t* __restrict__ bcnt, int scanned,
-                                                         int64_t* __restrict__ d_U, int64_t* __restrict__ n_unique,
-                                                         int64_t* __restrict__ uniq, int64_t* __restrict__ seg_start,
-                                                         int32_t* __restrict__ seg_occ0,
-                                                         int64_t* __restrict__ inverse) {
-  const int64_t base = (int64_t)blockIdx.x * kSegBlock * ITEMS + threadIdx.x;
-  // heads in earlier positions of the tile's earlier rounds
-  int64_t before = scanned ? bcnt[blockIdx.x] : block_offset(bcnt, blockIdx.x);
-  for (int r = 0; r < ITEMS; ++r) {
-    const int64_t i = base + (int64_t)r * kSegBlock;
-    const int f = is_head(sk, i, n);
-    int v[1] = {f}, ex[1], tot[1];
-    block_excl_scan<kSegBlock, 1>(v, ex, tot);
-    const int64_t u = before + ex[0] + f - 1;   // segment of position i
-    if (i < n) {
-      const int32_t o = sv[i];
-      if (f) {
-        uniq[u] = (int64_t)sk[i];
-        seg_start[u] = i;
-        seg_occ0[u] = o;
-      }
-      if (inverse && o >= 0 && o < n) inverse[o] = u;
-    }
-    before += tot[0];
-    __syncthreads();   // block_excl_scan's LDS is reused by the next round
-  }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-    *d_U = before;
-    if (n_unique) *n_unique = before;
-    seg_start[before] = n;
-  }
 }
 
 // Sort path.  A segment of more than kHotLen occurrences is hot: the partial-chunk kernel sums all of its runs (its
@@ -353,55 +403,163 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__
 __device__ __forceinline__ int part_chunks(int64_t L) {
   return (int)(seg_hot(L) ? (L + kSegChunk - 1) / kSegChunk : (L - 1) / kSegChunk);
 }
-__device__ __forceinline__ int extra_chunks(const int64_t* __restrict__ seg_start, int64_t u, int64_t U) {
-  return u < U ? part_chunks(seg_start[u + 1] - seg_start[u]) : 0;
-}
 
-// Partial chunks of each segment: per-block counts.  Also clears the hot-segment count.
-template <int ITEMS>
-__global__ __launch_bounds__(kSegBlock) void k_chunk_count(const int64_t* __restrict__ seg_start,
-                                                           const int64_t* __restrict__ d_U,
-                                                           int64_t* __restrict__ bsum, int64_t* __restrict__ d_hot) {
-  const int64_t base = (int64_t)blockIdx.x * kSegBlock * ITEMS + threadIdx.x;
-  const int64_t U = *d_U;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *d_hot = 0;
-  int v[1] = {0}, ex[1], tot[1];
-  for (int r = 0; r < ITEMS; ++r) v[0] += extra_chunks(seg_start, base + (int64_t)r * kSegBlock, U);
-  block_excl_scan<kSegBlock, 1>(v, ex, tot);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = tot[0];
-}
-
-// chunk_off[u] = first work item of segment u's partial chunks; chunk_seg[item] = u; hot segments are listed in
-// hot_list[0 .. *d_hot) (in no particular order: each is summed on its own).  The block's first work item is the sum
-// of the earlier blocks' counts (k_chunk_count), or bcnt[block] with `scanned`; the last block stores the number of
-// work items to *d_E.
-template <int ITEMS>
-__global__ __launch_bounds__(kSegBlock) void k_chunk_apply(const int64_t* __restrict__ seg_start,
-                                                           const int64_t* __restrict__ d_U,
-                                                           const int64_t* __restrict__ bcnt, int scanned,
-                                                           int32_t* __restrict__ chunk_off,
-                                                           int32_t* __restrict__ chunk_seg,
-                                                           int32_t* __restrict__ hot_list,
-                                                           int64_t* __restrict__ d_hot, int64_t* __restrict__ d_E) {
-  const int64_t base = (int64_t)blockIdx.x * kSegBlock * ITEMS + threadIdx.x;
-  const int64_t U = *d_U;
-  int64_t before = scanned ? bcnt[blockIdx.x] : block_offset(bcnt, blockIdx.x);
+// Segment heads: unique ids, segment starts, each segment's first occurrence index and the inverse, and (hot_list not
+// NULL) the segments of more than hot_len occurrences in hot_list[0 .. *d_hot) and, with chunk_off, the partial-chunk
+// plan: chunk_off[u] = first work item of segment u's partial chunks, for the segments that have any, and
+// chunk_seg[item] = u.  The block's first segment index
+// is the sum of the earlier blocks' head counts (k_seg_count), or, with `scanned`, bcnt[block] after k_scan_blocks.
+// The last block stores U to d_U (and n_unique) and seg_start[U] = n.
+//
+// A segment's length, which decides its chunks, is the distance to the next head: in its round's mask, in a later
+// round's or wave's, or in a later tile (bfirst).  The work items of a block's chunks are reserved with one atomic
+// add, so their order over the segments is not fixed; no sum depends on it (each group sum has its own parts row).
+// One launch in place of three (heads with a block scan per round, chunk counts, chunk plan): 28 us against 20 + 8 +
+// 20 and two scan launches of 4.5 at config C3's 3.4M positions, 10 against 18 + 8 + 21 at C5's 426k.
+template <typename Key, int ITEMS>
+__global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__ sk, const int32_t* __restrict__ sv,
+                                                         int64_t n, const int64_t* __restrict__ bcnt, int scanned,
+                                                         const int32_t* __restrict__ bfirst,
+                                                         int64_t* __restrict__ d_U, int64_t* __restrict__ n_unique,
+                                                         int64_t* __restrict__ uniq, int64_t* __restrict__ seg_start,
+                                                         int32_t* __restrict__ seg_occ0,
+                                                         int64_t* __restrict__ inverse,
+                                                         int32_t* __restrict__ chunk_off,
+                                                         int32_t* __restrict__ chunk_seg,
+                                                         int32_t* __restrict__ hot_list, int hot_len,
+                                                         int64_t* __restrict__ d_hot, int64_t* __restrict__ d_E) {
+  __shared__ int wcnt[kSegWaves], wext[kSegWaves], whot[kSegWaves];
+  __shared__ int wfirst[kSegWaves];
+  __shared__ int64_t res[2];
+  const int lane = threadIdx.x & 63, w = block_wave();
+  const int64_t nblk = gridDim.x, p0 = ((int64_t)blockIdx.x * kSegWaves + w) * (64 * ITEMS);
+  Key kk[ITEMS];
+  int32_t vv[ITEMS];
+  uint64_t hm[ITEMS];
+#pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
-    const int64_t u = base + (int64_t)r * kSegBlock;
-    const int e = extra_chunks(seg_start, u, U);
-    int v[1] = {e}, ex[1], tot[1];
-    block_excl_scan<kSegBlock, 1>(v, ex, tot);
-    if (u < U) {
-      const int64_t off = before + ex[0];
-      chunk_off[u] = (int32_t)off;
-      for (int c = 0; c < e; ++c) chunk_seg[off + c] = (int32_t)u;
-      if (seg_hot(seg_start[u + 1] - seg_start[u]))
-        hot_list[atomicAdd(reinterpret_cast<unsigned long long*>(d_hot), 1ull)] = (int32_t)u;
-    }
-    before += tot[0];
-    __syncthreads();
+    const int64_t i = p0 + r * 64 + lane;
+    vv[r] = i < n ? sv[i] : -1;
   }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_E = before;
+  seg_heads<Key, ITEMS>(sk, p0, n, kk, hm);
+  // the first head past this tile (n: none)
+  int nxt = (int)n;
+  for (int64_t b0 = (int64_t)blockIdx.x + 1; b0 < nblk; b0 += 64) {
+    const int f = b0 + lane < nblk ? bfirst[b0 + lane] : (int)n;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(f < n);
+    if (m) {
+      nxt = lane_value(f, __builtin_ctzll(m));
+      break;
+    }
+  }
+  int c = 0;
+  int first = (int)n;
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    c += __builtin_popcountll(hm[r]);
+    if (hm[r]) first = (int)p0 + r * 64 + __builtin_ctzll(hm[r]);
+  }
+  if (lane == 0) {
+    wcnt[w] = c;
+    wfirst[w] = first;
+  }
+  const int64_t before = scanned ? bcnt[blockIdx.x] : block_offset(bcnt, blockIdx.x);
+  __syncthreads();
+  int64_t run = before, tot = before;   // heads before this wave, and through this block
+#pragma unroll
+  for (int v = 0; v < kSegWaves; ++v) {
+    run += v < w ? wcnt[v] : 0;
+    tot += wcnt[v];
+  }
+#pragma unroll
+  for (int v = kSegWaves - 1; v >= 0; --v)
+    if (v > w && wfirst[v] < n) nxt = __builtin_amdgcn_readfirstlane(wfirst[v]);
+  if (blockIdx.x == nblk - 1 && threadIdx.x == 0) {
+    *d_U = tot;
+    if (n_unique) *n_unique = tot;
+    seg_start[tot] = n;
+  }
+  // the segments and the inverse; the lengths of this wave's segments, last round first
+  int64_t end = run + c;      // segments through the round
+  int ext = 0, hot = 0;       // this lane's partial chunks and hot segments
+  uint32_t has = 0;           // rounds with a hot segment or one of more than one chunk (wave-uniform)
+  int after[ITEMS];           // first head past each round
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    const int64_t i = p0 + r * 64 + lane;
+    const uint64_t m = hm[r];
+    const bool head = (m >> lane) & 1;
+    const int64_t u0 = end - __builtin_popcountll(m);   // segments before the round
+    const int64_t u = u0 + __builtin_popcountll(m & lanemask_lt()) + (head ? 0 : -1);
+    after[r] = nxt;
+    if (head) {
+      uniq[u] = (int64_t)kk[r];
+      seg_start[u] = i;
+      seg_occ0[u] = vv[r];
+    }
+    if (inverse && vv[r] >= 0 && vv[r] < n) inverse[vv[r]] = u;
+    if (hot_list) {
+      const uint64_t up = lane == 63 ? 0ull : m >> (lane + 1);
+      const int64_t L = head ? (up ? (int64_t)__builtin_ctzll(up) + 1 : (int64_t)nxt - i) : 1;
+      const int e = chunk_off ? part_chunks(L) : 0;
+      ext += e;
+      hot += L > hot_len ? 1 : 0;
+      has |= __builtin_amdgcn_ballot_w64(e > 0 || L > hot_len) ? 1u << r : 0u;
+    }
+    if (m) nxt = (int)p0 + r * 64 + __builtin_ctzll(m);
+    end = u0;
+  }
+  if (!hot_list) return;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    ext += __shfl_xor(ext, d, 64);
+    hot += __shfl_xor(hot, d, 64);
+  }
+  if (lane == 0) {
+    wext[w] = ext;
+    whot[w] = hot;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    int64_t x = 0;
+    for (int v = 0; v < kSegWaves; ++v) x += threadIdx.x ? whot[v] : wext[v];
+    res[threadIdx.x] = x ? (int64_t)atomicAdd(reinterpret_cast<unsigned long long*>(threadIdx.x ? d_hot : d_E),
+                                              (unsigned long long)x)
+                         : 0;
+  }
+  __syncthreads();
+  if (!has) return;
+  int64_t eat = res[0], hat = res[1];
+  for (int v = 0; v < w; ++v) {
+    eat += wext[v];
+    hat += whot[v];
+  }
+  end = run + c;
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    const uint64_t m = hm[r];
+    const int64_t u0 = end - __builtin_popcountll(m);
+    end = u0;
+    if (!((has >> r) & 1u)) continue;
+    const int64_t i = p0 + r * 64 + lane;
+    const bool head = (m >> lane) & 1;
+    const int32_t u = (int32_t)(u0 + __builtin_popcountll(m & lanemask_lt()));
+    const uint64_t up = lane == 63 ? 0ull : m >> (lane + 1);
+    const int64_t L = head ? (up ? (int64_t)__builtin_ctzll(up) + 1 : (int64_t)after[r] - i) : 1;
+    const int e = chunk_off ? part_chunks(L) : 0, inc = wave_incl_scan<int>(e);
+    if (e > 0) chunk_off[u] = (int32_t)(eat + inc - e);
+    // the wave writes each segment's work items together (a hot segment has thousands)
+    for (uint64_t q = __builtin_amdgcn_ballot_w64(e > 0); q; q &= q - 1) {
+      const int l = __builtin_ctzll(q);
+      const int qe = lane_value(e, l), qu = lane_value(u, l);
+      const int64_t qo = eat + lane_value(inc - e, l);
+      for (int k = lane; k < qe; k += 64) chunk_seg[qo + k] = qu;
+    }
+    eat += lane_value(inc, 63);
+    const uint64_t hb = __builtin_amdgcn_ballot_w64(L > hot_len);
+    if (L > hot_len) hot_list[hat + __builtin_popcountll(hb & lanemask_lt())] = u;
+    hat += __builtin_popcountll(hb);
+  }
 }
 
 // ---- dedup plan of a batch laid out by field -------------------------------------------------------------------
@@ -836,6 +994,214 @@ __global__ __launch_bounds__(256) void k_seg_final(const float* __restrict__ gra
   }
 }
 
+// Adam on a lane's chunks: adam_elem's operations with one range check for all of them (frag_adam).
+template <int NC>
+__device__ __forceinline__ void chunk_adam(ChunkFrag<NC>& w, ChunkFrag<NC>& m, ChunkFrag<NC>& v,
+                                           const ChunkFrag<NC>& g, const AdamScalars& s) {
+  RowFrag<4 * NC> fw, fm, fv, fg;
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      fw.v[4 * c + j] = w.v[c][j];
+      fm.v[4 * c + j] = m.v[c][j];
+      fv.v[4 * c + j] = v.v[c][j];
+      fg.v[4 * c + j] = g.v[c][j];
+    }
+  frag_adam<4 * NC>(fw, fm, fv, fg, s);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w.v[c][j] = fw.v[4 * c + j];
+      m.v[c][j] = fm.v[4 * c + j];
+      v.v[c][j] = fv.v[4 * c + j];
+    }
+}
+
+// The final sums (and Adam, MODE 1) in the chunk layout (elr_seg_dev.h): LPR lanes per segment, 64 / LPR segments per
+// wave, WIN: ATen's windowed order.  A one-occurrence segment, the common case, costs two dependent round trips (its
+// metadata; its gradient row and state), and a longer one two more per kSubRows occurrences.  The first hot_blocks
+// blocks take the segments of hot_list, one each at a time: the whole block loads the run sums (windowed: the
+// gradients) into LDS, kSubStage floats of them, and one group adds them in order.  Against a wave per segment with
+// 4 bytes a lane: 26 us
+// against 37 at 107k occurrences, 40k segments of width 48 (most of it the dependent round trips of the 60-occurrence
+// segments: 12 without them).
+template <int NC>
+constexpr int kSubRows = NC == 1 ? kAtenGroup : kAtenGroup / 2;
+constexpr int kSubStage = 4096;   // floats: 16 KB, so that LDS leaves the wave count alone
+template <int LPR, int NC, int MODE, bool WIN>
+struct SegFinalSub {
+  const float* grad;
+  int64_t D;
+  const int32_t* sv;
+  const int64_t* seg_start;
+  const int32_t* seg_occ0;
+  const int64_t* uniq;
+  const int32_t* chunk_off;
+  const float* parts;
+  const int64_t* d_U;
+  int64_t u_base;
+  const int32_t* hot_list;
+  const int64_t* d_hot;
+  int64_t hot_blocks;
+  float* out;
+  int64_t nrows;
+  AdamScalars s;
+  __device__ void operator()(int64_t block, int64_t nblocks) const;
+  __device__ void hot(int64_t block) const;
+  __device__ __forceinline__ void emit(int64_t row, int l, int nchunk, const ChunkFrag<NC>& tot) const;
+};
+
+template <int LPR, int NC, int MODE, bool WIN>
+__device__ __forceinline__ void SegFinalSub<LPR, NC, MODE, WIN>::emit(int64_t row, int l, int nchunk,
+                                                                      const ChunkFrag<NC>& tot) const {
+  if (MODE == 0) {
+    chunk_store<LPR, NC>(out + row * D, l, nchunk, tot);
+  } else {
+    float* rec = out + row * 3 * D;
+    ChunkFrag<NC> w = chunk_load<LPR, NC, false>(rec, l, nchunk),
+                  m = chunk_load<LPR, NC, false>(rec + D, l, nchunk),
+                  v = chunk_load<LPR, NC, false>(rec + 2 * D, l, nchunk);
+    chunk_adam<NC>(w, m, v, tot, s);
+    chunk_store<LPR, NC>(rec, l, nchunk, w);
+    chunk_store<LPR, NC>(rec + D, l, nchunk, m);
+    chunk_store<LPR, NC>(rec + 2 * D, l, nchunk, v);
+  }
+}
+
+template <int LPR, int NC, int MODE, bool WIN>
+__device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
+  __shared__ f32x4 stage[kSubStage / 4];
+  __shared__ int32_t win[WIN ? kSubStage / 4 : 1];   // windowed: the staged rows' windows
+  const int t = threadIdx.x, nchunk = (int)(D / 4), per = (kSubStage / 4) / nchunk;
+  const int64_t nh = *d_hot;
+  for (int64_t h = block; h < nh; h += hot_blocks) {
+    const int64_t u = hot_list[h], s0 = seg_start[u], L = seg_start[u + 1] - s0;
+    const int64_t nr = WIN ? L : (L + kAtenGroup - 1) / kAtenGroup;   // rows to add: gradients, or run sums
+    const f32x4* src = reinterpret_cast<const f32x4*>(
+        WIN ? grad : parts + (int64_t)chunk_off[u] * kGroupsPerChunk * D);
+    ChunkFrag<NC> tot = chunk_zero<NC>(), acc = tot;
+    int32_t prev = -1;
+    for (int64_t r0 = 0; r0 < nr; r0 += per) {
+      const int m = (int)(nr - r0 < per ? nr - r0 : per);
+      __syncthreads();
+      for (int q = t; q < m * nchunk; q += 256) {
+        const int r = q / nchunk;
+        const int64_t row = WIN ? (int64_t)sv[s0 + r0 + r] : r0 + r;
+        if (WIN && q - r * nchunk == 0) win[r] = (int32_t)(row >> kAtenWinShift);
+        stage[q] = src[row * nchunk + (q - r * nchunk)];
+      }
+      __syncthreads();
+      if (t < LPR) {
+        for (int r = 0; r < m; ++r) {
+          ChunkFrag<NC> x;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            const f32x4 g = t + c * LPR < nchunk ? stage[r * nchunk + t + c * LPR] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x.v[c][j] = g[j];
+          }
+          if (!WIN) {
+            chunk_add<NC>(tot, x);
+          } else if (win[r] != prev) {
+            if (prev >= 0) chunk_add<NC>(tot, acc);
+            acc = x;
+            prev = win[r];
+          } else {
+            chunk_add<NC>(acc, x);
+          }
+        }
+      }
+    }
+    if (t < LPR) {
+      if (WIN) chunk_add<NC>(tot, acc);
+      const int64_t row = uniq ? uniq[u] : u;
+      if (row >= 0 && row < nrows) emit(row, t, nchunk, tot);
+    }
+  }
+}
+
+template <int LPR, int NC, int MODE, bool WIN>
+__device__ void SegFinalSub<LPR, NC, MODE, WIN>::operator()(int64_t block, int64_t) const {
+  if (block < hot_blocks) {
+    hot(block);
+    return;
+  }
+  constexpr int GPW = 64 / LPR;
+  const int lane = threadIdx.x & 63, l = lane & (LPR - 1);
+  const int nchunk = (int)(D / 4);
+  const int64_t u = u_base + ((block - hot_blocks) * 4 + (threadIdx.x >> 6)) * GPW + lane / LPR;
+  if (u >= *d_U) return;
+  const int64_t s0 = seg_start[u], L = seg_start[u + 1] - s0;
+  const int64_t row = uniq ? uniq[u] : u;   // NULL: segment u goes to row u
+  const int32_t o0 = seg_occ0[u];
+  if (row < 0 || row >= nrows || (WIN ? L > kWinHot : seg_hot(L))) return;   // hot segments: a block's
+  ChunkFrag<NC> acc = chunk_load<LPR, NC, true>(grad + (int64_t)o0 * D, l, nchunk);
+  float* rec = out + row * 3 * D;
+  ChunkFrag<NC> w, m, v;
+  if (MODE == 1) {
+    w = chunk_load<LPR, NC, false>(rec, l, nchunk);
+    m = chunk_load<LPR, NC, false>(rec + D, l, nchunk);
+    v = chunk_load<LPR, NC, false>(rec + 2 * D, l, nchunk);
+  }
+  const int inl = (int)(WIN ? L : (L < kSegChunk ? L : kSegChunk));
+  ChunkFrag<NC> tot = chunk_zero<NC>();
+  int32_t prev = o0;
+  int in_run = 1;   // occurrences of the open run (sort path)
+  constexpr int R = kSubRows<NC>;
+  int32_t o[R];
+#pragma unroll
+  for (int e = 0; e < R; ++e) o[e] = sv[s0 + (1 + e < inl ? 1 + e : 0)];
+  for (int k0 = 1; k0 < inl; k0 += R) {
+    // this batch's rows, then the next batch's indices, so that a batch costs one round trip
+    ChunkFrag<NC> g[R];
+    int32_t on[R];
+#pragma unroll
+    for (int e = 0; e < R; ++e) g[e] = chunk_load<LPR, NC, true>(grad + (int64_t)o[e] * D, l, nchunk);
+#pragma unroll
+    for (int e = 0; e < R; ++e) on[e] = sv[s0 + (k0 + R + e < inl ? k0 + R + e : 0)];
+#pragma unroll
+    for (int e = 0; e < R; ++e) {
+      if (k0 + e >= inl) continue;
+      const bool head = WIN ? (o[e] >> kAtenWinShift) != (prev >> kAtenWinShift) : in_run == kAtenGroup;
+      if (head) {
+        chunk_add<NC>(tot, acc);
+        acc = g[e];
+        in_run = 1;
+      } else {
+        chunk_add<NC>(acc, g[e]);
+        ++in_run;
+      }
+      prev = o[e];
+    }
+#pragma unroll
+    for (int e = 0; e < R; ++e) o[e] = on[e];
+  }
+  chunk_add<NC>(tot, acc);
+  if (!WIN && L > kSegChunk) {
+    const int np = (int)((L - kSegChunk + kAtenGroup - 1) / kAtenGroup);
+    const float* pr = parts + (int64_t)chunk_off[u] * kGroupsPerChunk * D;
+    for (int c0 = 0; c0 < np; c0 += kSubRows<NC>) {
+      ChunkFrag<NC> pc[kSubRows<NC>];
+#pragma unroll
+      for (int e = 0; e < kSubRows<NC>; ++e)
+        pc[e] = chunk_load<LPR, NC, false>(pr + (int64_t)(c0 + e < np ? c0 + e : c0) * D, l, nchunk);
+#pragma unroll
+      for (int e = 0; e < kSubRows<NC>; ++e)
+        if (c0 + e < np) chunk_add<NC>(tot, pc[e]);
+    }
+  }
+  if (MODE == 0) {
+    chunk_store<LPR, NC>(out + row * D, l, nchunk, tot);
+  } else {
+    chunk_adam<NC>(w, m, v, tot, s);
+    chunk_store<LPR, NC>(rec, l, nchunk, w);
+    chunk_store<LPR, NC>(rec + D, l, nchunk, m);
+    chunk_store<LPR, NC>(rec + 2 * D, l, nchunk, v);
+  }
+}
+
 // Wave-per-row form of k_seg_final for D = 64*VPL (lane l holds floats [l*VPL, l*VPL + VPL)): no grid-stride
 // loop, each wave owns kSegPerWave consecutive segments starting at u_base + wave * kSegPerWave; waves past U exit.
 // All per-segment metadata (bounds, row id, first occurrence) are scalar loads issued together, then the first
@@ -1093,13 +1459,20 @@ __global__ __launch_bounds__(256) void k_seg_final_wpr(SegFinalWpr<VPL, MODE> f)
 // ---- host side -------------------------------------------------------------------------------------------------
 inline int64_t al256(int64_t b) { return (b + 255) & ~int64_t(255); }
 
+// ATen's windowed order applies up to kAtenSmall indices: returns the window's shift there, 0 on the sort path.
+inline int win_shift_for(int64_t n) { return n <= kAtenSmall ? kAtenWinShift : 0; }
+// Bound of the hot segments of n occurrences (and the blocks that take them).
+inline int64_t hot_max(int64_t n) { return n / (win_shift_for(n) ? kWinHot : kHotLen) + 1; }
+
 // Scratch carve-up for n occurrences of width D.
 struct DedupScratch {
   void* keys[2];
   int32_t* vals[2];
-  int64_t* hist;      // [kRadixMaxBins * ntile], ntile = n / (kSortThreads * items_for(n)) rounded up
-  int64_t* dtot;      // [256] digit totals
-  int64_t* bsum;      // [n / (kSegBlock * items_for(n)) + 1]
+  int32_t* hist;      // [kRadixMaxBins * ntile] digit counts per sort tile (sort_tiles)
+  int32_t* dtot;      // [kRadixMaxBins] digit totals
+  int64_t* fcnt;      // [2 * kFieldMax] segments and chunks of each field (elr_dedup_plan_fields)
+  int64_t* bsum;      // [n / (kSegBlock * seg_items_for(n)) + 1] heads per segment tile
+  int32_t* bfirst;    // the same count: each tile's first head
   int64_t* d_tot;     // [3]: U, E (partial chunks), hot segments
   int64_t* uniq;      // [n]
   int64_t* seg_start; // [n + 1]
@@ -1107,11 +1480,16 @@ struct DedupScratch {
   int32_t* chunk_off; // [n]
   int32_t* chunk_seg; // [nch]: n / kSegChunk + n / kHotLen + 2 bounds the partial chunks
   float* parts;       // [nch * kGroupsPerChunk * D] group sums of the partial chunks
-  int32_t* hot_list;  // [n / kHotLen + 1] hot segments
+  int32_t* hot_list;  // [hot_max(n)] hot segments
 };
 
+// (the segment tiles' counts, at most kSegPerSort tiles per sort tile, fit beside the digit counts, and the fields'
+// counts beside the digit totals)
+constexpr int64_t kSegPerSort = kSortTile / (kSegBlock * kSegItemsSmall);
+static_assert(kSegPerSort * 12 <= kRadixMaxBins * 4 && 2 * kFieldMax * 8 <= kRadixMaxBins * 4, "shared scratch");
+
 inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void* base) {
-  const int64_t ntile = cdiv(n, kSortThreads * items_for(n)), nblk = cdiv(n, kSegBlock * items_for(n));
+  const int64_t ntile = sort_tiles(n), nblk = cdiv(n, kSegBlock * seg_items_for(n));
   const int64_t nch = n / kSegChunk + n / kHotLen + 2;
   int64_t o = 0;
   char* b = (char*)base;
@@ -1125,9 +1503,13 @@ inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void
   s.keys[1] = take(n * 8);
   s.vals[0] = (int32_t*)take(n * 4);
   s.vals[1] = (int32_t*)take(n * 4);
-  s.hist = (int64_t*)take(kRadixMaxBins * ntile * 8);
-  s.dtot = (int64_t*)take(kRadixMaxBins * 8);
-  s.bsum = (int64_t*)take(nblk * 8);
+  // the digit counts, then the segment tiles' counts; the digit totals, then the fields' counts
+  s.hist = (int32_t*)take(kRadixMaxBins * ntile * 8);
+  s.bsum = (int64_t*)(s.hist + kRadixMaxBins * ntile);
+  s.bfirst = (int32_t*)(s.bsum + nblk);
+  s.dtot = (int32_t*)take(kRadixMaxBins * 8);
+  s.fcnt = (int64_t*)(s.dtot + kRadixMaxBins);
+  o += al256(ntile * 8);   // unused: keeps the largest n of elr_adam_dedup_noalloc where it has been
   s.d_tot = (int64_t*)take(3 * 8);
   s.uniq = (int64_t*)take(n * 8);
   s.seg_start = (int64_t*)take((n + 1) * 8);
@@ -1135,7 +1517,7 @@ inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void
   s.chunk_off = (int32_t*)take(n * 4);
   s.chunk_seg = (int32_t*)take(nch * 4);
   s.parts = (float*)take(nch * kGroupsPerChunk * D * 4);
-  s.hot_list = (int32_t*)take((n / kHotLen + 1) * 4);
+  s.hot_list = (int32_t*)take(hot_max(n) * 4);
   if (out) *out = s;
   return o;
 }
@@ -1152,30 +1534,34 @@ inline int sort_passes(int key_bits) {
   return passes;
 }
 
-// One pass over RB-bit digit p of the keys: histogram, scan, stable scatter from buffer cur (the caller's ids on
-// the first pass) to buffer nxt.
-template <typename Key, int ITEMS, int RB>
-static void radix_pass(const int64_t* ids, int64_t n, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
-  const int64_t ntile = cdiv(n, kSortThreads * ITEMS);
-  const int shift = RB * p;
+// One pass over RB-bit digit p of the keys: histogram, scan (or none: fold), stable scatter from buffer cur (the
+// caller's ids on the first pass) to buffer nxt.
+template <typename Key, int RB, int NT>
+static void radix_pass_nt(const int64_t* ids, int64_t n, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
+  const int64_t ntile = sort_tiles(n);
+  const int shift = RB * p, fold = ntile <= kSortFoldTiles;
+  const unsigned grid = (unsigned)ntile;
   constexpr int BINS = 1 << RB;
-  constexpr unsigned kScanGrid = (unsigned)(BINS / (kSortThreads / 64));   // a wave per digit
+  constexpr unsigned kScanGrid = (unsigned)(BINS / (kHistScanThreads / 64));   // a wave per digit
   Key* kb[2] = {(Key*)S.keys[0], (Key*)S.keys[1]};
-  if (p == 0) {
-    k_radix_hist<int64_t, Key, ITEMS, RB><<<(unsigned)ntile, kSortThreads, 0, st>>>(ids, n, shift, S.hist, ntile);
-    k_radix_hist_scan<<<kScanGrid, kSortThreads, 0, st>>>(S.hist, ntile, BINS, S.dtot);
-    k_radix_scatter<int64_t, Key, true, ITEMS, RB><<<(unsigned)ntile, kSortThreads, 0, st>>>(
-        ids, nullptr, n, shift, S.hist, S.dtot, ntile, kb[nxt], S.vals[nxt]);
-  } else {
-    k_radix_hist<Key, Key, ITEMS, RB><<<(unsigned)ntile, kSortThreads, 0, st>>>(kb[cur], n, shift, S.hist, ntile);
-    k_radix_hist_scan<<<kScanGrid, kSortThreads, 0, st>>>(S.hist, ntile, BINS, S.dtot);
-    k_radix_scatter<Key, Key, false, ITEMS, RB><<<(unsigned)ntile, kSortThreads, 0, st>>>(
-        kb[cur], S.vals[cur], n, shift, S.hist, S.dtot, ntile, kb[nxt], S.vals[nxt]);
-  }
+  if (p == 0) k_radix_hist<int64_t, Key, RB, NT><<<grid, NT, 0, st>>>(ids, n, shift, S.hist, ntile, fold);
+  else k_radix_hist<Key, Key, RB, NT><<<grid, NT, 0, st>>>(kb[cur], n, shift, S.hist, ntile, fold);
+  if (!fold) k_radix_hist_scan<<<kScanGrid, kHistScanThreads, 0, st>>>(S.hist, ntile, BINS, S.dtot);
+  if (p == 0)
+    k_radix_scatter<int64_t, Key, true, RB, NT><<<grid, NT, 0, st>>>(ids, nullptr, n, shift, S.hist, S.dtot, (int)ntile,
+                                                                      fold, kb[nxt], S.vals[nxt]);
+  else
+    k_radix_scatter<Key, Key, false, RB, NT><<<grid, NT, 0, st>>>(kb[cur], S.vals[cur], n, shift, S.hist, S.dtot,
+                                                                   (int)ntile, fold, kb[nxt], S.vals[nxt]);
+}
+template <typename Key, int RB>
+static void radix_pass(const int64_t* ids, int64_t n, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
+  if (n >= kSortBig) radix_pass_nt<Key, RB, kSortThreadsBig>(ids, n, p, cur, nxt, S, st);
+  else radix_pass_nt<Key, RB, kSortThreadsSmall>(ids, n, p, cur, nxt, S, st);
 }
 
 // Sort (ids, positions) by id; returns which buffer holds the result.
-template <typename Key, int ITEMS>
+template <typename Key>
 static int radix_sort(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, hipStream_t st) {
   int passes, rb;
   sort_plan(key_bits, max_digit_bits<Key>(), passes, rb);
@@ -1184,62 +1570,46 @@ static int radix_sort(const int64_t* ids, int64_t n, int key_bits, DedupScratch&
     const int nxt = p == 0 ? 0 : cur ^ 1;
     if constexpr (max_digit_bits<Key>() >= 10) {
       if (rb == 10) {
-        radix_pass<Key, ITEMS, 10>(ids, n, p, cur, nxt, S, st);
+        radix_pass<Key, 10>(ids, n, p, cur, nxt, S, st);
         cur = nxt;
         continue;
       }
     }
-    if (rb == 9) radix_pass<Key, ITEMS, 9>(ids, n, p, cur, nxt, S, st);
-    else radix_pass<Key, ITEMS, 8>(ids, n, p, cur, nxt, S, st);
+    if (rb == 9) radix_pass<Key, 9>(ids, n, p, cur, nxt, S, st);
+    else radix_pass<Key, 8>(ids, n, p, cur, nxt, S, st);
     cur = nxt;
   }
   return cur;
 }
 
-// Sort, segment heads (uniq / seg_start / inverse, U in d_tot[0]) and the extra-chunk plan (E in d_tot[1]).
+// Segment heads (uniq / seg_start / inverse, U in d_tot[0]) of the sorted keys and, for segment sums (sums), the hot
+// segments and the partial-chunk plan (E in d_tot[1]; the windowed path has no partial chunks).
 template <typename Key, int ITEMS>
-static int dedup_core_items(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, int64_t* uniq_out,
-                            int64_t* inverse, int64_t* n_unique, hipStream_t st) {
-  const int cur = radix_sort<Key, ITEMS>(ids, n, key_bits, S, st);
-  const Key* sk = (const Key*)S.keys[cur];
-  const int32_t* sv = S.vals[cur];
+static void seg_plan(const Key* sk, const int32_t* sv, int64_t n, DedupScratch& S, int64_t* uniq, int64_t* inverse,
+                     int64_t* n_unique, bool sums, hipStream_t st) {
   const int64_t nblk = cdiv(n, kSegBlock * ITEMS);
-  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
   const int scanned = nblk > kFoldMaxBlocks;
-  k_seg_count<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(sk, n, S.bsum);
+  k_seg_count<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(sk, n, S.bsum, S.bfirst, S.d_tot + 1, S.d_tot + 2);
   if (scanned) k_scan_blocks<<<1, kScanBlock, 0, st>>>(S.bsum, nblk);
-  k_seg_apply<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(sk, sv, n, S.bsum, scanned, S.d_tot, n_unique, uniq,
-                                                                S.seg_start, S.seg_occ0, inverse);
-  return cur;
+  k_seg_apply<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(
+      sk, sv, n, S.bsum, scanned, S.bfirst, S.d_tot, n_unique, uniq, S.seg_start, S.seg_occ0, inverse,
+      win_shift_for(n) ? nullptr : S.chunk_off, S.chunk_seg, sums ? S.hot_list : nullptr,
+      (int)(win_shift_for(n) ? kWinHot : kHotLen), S.d_tot + 2, S.d_tot + 1);
 }
 
+// Sort, segment heads and partial-chunk plan; returns which buffer holds the sorted positions.
 template <typename Key>
 static int dedup_core(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, int64_t* uniq_out,
-                      int64_t* inverse, int64_t* n_unique, hipStream_t st) {
-  return items_for(n) == kItemsBig
-             ? dedup_core_items<Key, kItemsBig>(ids, n, key_bits, S, uniq_out, inverse, n_unique, st)
-             : dedup_core_items<Key, kItemsSmall>(ids, n, key_bits, S, uniq_out, inverse, n_unique, st);
+                      int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
+  const int cur = radix_sort<Key>(ids, n, key_bits, S, st);
+  const Key* sk = (const Key*)S.keys[cur];
+  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
+  if (seg_items_for(n) == kSegItemsBig)
+    seg_plan<Key, kSegItemsBig>(sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
+  else
+    seg_plan<Key, kSegItemsSmall>(sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
+  return cur;
 }
-
-// ATen's windowed order applies up to kAtenSmall indices: returns the window's shift there, 0 on the sort path.
-inline int win_shift_for(int64_t n) { return n <= kAtenSmall ? kAtenWinShift : 0; }
-
-template <int ITEMS>
-static void chunk_plan_items(int64_t n, DedupScratch& S, hipStream_t st) {
-  const int64_t nblk = cdiv(n, kSegBlock * ITEMS);
-  const int scanned = nblk > kFoldMaxBlocks;
-  k_chunk_count<ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(S.seg_start, S.d_tot, S.bsum, S.d_tot + 2);
-  if (scanned) k_scan_blocks<<<1, kScanBlock, 0, st>>>(S.bsum, nblk);
-  k_chunk_apply<ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(S.seg_start, S.d_tot, S.bsum, scanned, S.chunk_off,
-                                                             S.chunk_seg, S.hot_list, S.d_tot + 2, S.d_tot + 1);
-}
-
-static void chunk_plan(int64_t n, DedupScratch& S, hipStream_t st) {
-  if (win_shift_for(n)) return;   // the windowed path sums every segment in one wave: no extra chunks
-  if (items_for(n) == kItemsBig) chunk_plan_items<kItemsBig>(n, S, st);
-  else chunk_plan_items<kItemsSmall>(n, S, st);
-}
-
 
 template <int NQ>
 inline SegPartials<NQ> seg_partials_of(const float* grad, int64_t D, const int32_t* sv, const DedupScratch& S) {
@@ -1255,6 +1625,33 @@ static void seg_reduce(const float* grad, int64_t D, const int32_t* sv, DedupScr
                                                        ws, out, nrows, s);
 }
 
+// The chunk-layout form: partial chunks (sort path), then the final kernel in launches of at most 2^22 blocks (U <= n;
+// blocks past U exit at once), the first with a block per possible hot segment.
+template <int MODE>
+static void seg_reduce_sub(int lpr, const float* grad, int64_t D, const int32_t* sv, DedupScratch& S,
+                           const int64_t* uniq, int64_t n, float* out, int64_t nrows, const AdamScalars& s,
+                           hipStream_t st, bool partials) {
+  const bool win = win_shift_for(n) != 0;
+  if (!win && partials) {
+    const SegPartialsLaunch L{seg_partials_of<1>(grad, D, sv, S), seg_partials_blocks(n)};
+    seg_partials_visit(L, [&](const auto& f, int64_t nb) { launch1(f, nb, st); });
+  }
+  chunk_visit(lpr, D, [&](auto L_, auto N_) {
+    constexpr int LPR = L_.value, NC = N_.value, SPB = 4 * (64 / LPR);   // segments per block
+    const int64_t per = kOneShotBlocks * SPB;
+    for (int64_t a = 0; a < n; a += per) {
+      const int64_t m = n - a < per ? n - a : per, hb = a == 0 ? hot_max(n) : 0;
+      auto go = [&](const auto& f) { launch1(f, hb + cdiv(m, SPB), st); };
+      if (win)
+        go(SegFinalSub<LPR, NC, MODE, true>{grad, D, sv, S.seg_start, S.seg_occ0, uniq, S.chunk_off, S.parts, S.d_tot, a,
+                                            S.hot_list, S.d_tot + 2, hb, out, nrows, s});
+      else
+        go(SegFinalSub<LPR, NC, MODE, false>{grad, D, sv, S.seg_start, S.seg_occ0, uniq, S.chunk_off, S.parts, S.d_tot,
+                                             a, S.hot_list, S.d_tot + 2, hb, out, nrows, s});
+    }
+  });
+}
+
 template <int VPL, int MODE>
 static void seg_reduce_wpr(const float* grad, const int32_t* sv, DedupScratch& S, const int64_t* uniq, int64_t n,
                            float* out, int64_t nrows, const AdamScalars& s, hipStream_t st, bool partials) {
@@ -1265,7 +1662,7 @@ static void seg_reduce_wpr(const float* grad, const int32_t* sv, DedupScratch& S
   const int64_t per = kOneShotBlocks * 4 * kSegPerWave;
   for (int64_t a = 0; a < n; a += per) {
     const int64_t m = n - a < per ? n - a : per;
-    const int64_t hb = a == 0 ? n / kHotLen + 1 : 0;
+    const int64_t hb = a == 0 ? hot_max(n) : 0;
     const SegFinalWpr<VPL, MODE> f{grad, sv, S.seg_start, S.seg_occ0, uniq, S.chunk_off, S.parts, S.d_tot, a,
                                    S.hot_list, S.d_tot + 2, hb, out, nrows, s};
     k_seg_final_wpr<VPL, MODE><<<(unsigned)(hb + cdiv(m, 4 * kSegPerWave)), 256, 0, st>>>(f);
@@ -1276,7 +1673,9 @@ template <int MODE>
 static int seg_reduce_d(const float* grad, int64_t D, const int32_t* sv, DedupScratch& S, const int64_t* uniq,
                         int64_t n, float* out, int64_t nrows, const AdamScalars& s, hipStream_t st,
                         bool partials = true) {
-  if (aligned16(grad) && aligned16(out) && !win_shift_for(n)) {   // ATen's windowed order: the generic kernels
+  // a wave per row for D = 64, 128, 256 and 512 on the sort path, else rows in chunks of 16 bytes (the windowed order
+  // too), else (D % 4 != 0, unaligned arrays) a float per lane
+  if (aligned16(grad) && aligned16(out) && !win_shift_for(n)) {
     switch (D) {
       case 64: seg_reduce_wpr<1, MODE>(grad, sv, S, uniq, n, out, nrows, s, st, partials); return ELR_OK;
       case 128: seg_reduce_wpr<2, MODE>(grad, sv, S, uniq, n, out, nrows, s, st, partials); return ELR_OK;
@@ -1284,6 +1683,10 @@ static int seg_reduce_d(const float* grad, int64_t D, const int32_t* sv, DedupSc
       case 512: seg_reduce_wpr<8, MODE>(grad, sv, S, uniq, n, out, nrows, s, st, partials); return ELR_OK;
       default: break;
     }
+  }
+  if (const int lpr = chunk_lanes(D, grad, out)) {
+    seg_reduce_sub<MODE>(lpr, grad, D, sv, S, uniq, n, out, nrows, s, st, partials);
+    return ELR_OK;
   }
   const int64_t nq = cdiv(D, 64);
   switch (nq) {
@@ -1322,8 +1725,8 @@ extern "C" int elr_unique(const int64_t* ids, int64_t n, int key_bits, int64_t* 
   DedupScratch S;
   if (scratch_bytes < dedup_scratch_bytes(n, 1, &S, scratch)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
-  if (key_bits <= 32) dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, st);
-  else dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, st);
+  if (key_bits <= 32) dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, false, st);
+  else dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, false, st);
   return launch_status();
 }
 
@@ -1338,9 +1741,8 @@ extern "C" int elr_segment_sum(const float* grad, const int64_t* idx, int64_t n,
   if (scratch_bytes < dedup_scratch_bytes(n, D, &S, scratch)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
   const int kb = bits_for(num_rows);
-  const int cur = kb <= 32 ? dedup_core<uint32_t>(idx, n, kb, S, nullptr, nullptr, nullptr, st)
-                           : dedup_core<uint64_t>(idx, n, kb, S, nullptr, nullptr, nullptr, st);
-  chunk_plan(n, S, st);
+  const int cur = kb <= 32 ? dedup_core<uint32_t>(idx, n, kb, S, nullptr, nullptr, nullptr, true, st)
+                           : dedup_core<uint64_t>(idx, n, kb, S, nullptr, nullptr, nullptr, true, st);
   const AdamScalars none{};
   const int rc = seg_reduce_d<0>(grad, D, S.vals[cur], S, S.uniq, n, out, num_rows, none, st);
   return rc != ELR_OK ? rc : launch_status();
@@ -1358,9 +1760,8 @@ extern "C" int elr_adam_dedup(float* state, int64_t C, const int64_t* ids, const
   hipStream_t st = (hipStream_t)stream;
   const AdamScalars s = make_scalars(sc);
   const int kb = bits_for(C);
-  const int cur = kb <= 32 ? dedup_core<uint32_t>(ids, n, kb, S, nullptr, nullptr, nullptr, st)
-                           : dedup_core<uint64_t>(ids, n, kb, S, nullptr, nullptr, nullptr, st);
-  chunk_plan(n, S, st);
+  const int cur = kb <= 32 ? dedup_core<uint32_t>(ids, n, kb, S, nullptr, nullptr, nullptr, true, st)
+                           : dedup_core<uint64_t>(ids, n, kb, S, nullptr, nullptr, nullptr, true, st);
   const int rc = seg_reduce_d<1>(grad, D, S.vals[cur], S, S.uniq, n, state, C, s, st);
   return rc != ELR_OK ? rc : launch_status();
 }
@@ -1389,10 +1790,9 @@ extern "C" int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64
   DedupScratch S;
   if (plan_bytes < dedup_scratch_bytes(n, D, &S, plan)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
-  const int cur = key_bits <= 32 ? dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, st)
-                                 : dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, st);
+  const int cur = key_bits <= 32 ? dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, true, st)
+                                 : dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, true, st);
   if (cur != plan_result_buffer(key_bits)) return ELR_EINVAL;
-  chunk_plan(n, S, st);
   return launch_status();
 }
 
@@ -1415,7 +1815,6 @@ extern "C" int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t 
   if (!ids || !uniq || !n_unique || !plan) return ELR_EINVAL;
   DedupScratch S;
   if (plan_bytes < dedup_scratch_bytes(n, D, &S, plan)) return ELR_ECAPACITY;
-  static_assert(2 * kFieldMax <= kRadixMaxBins, "the per-field counts fit in the first histogram's space");
   FieldBounds fb;
   for (int64_t c = 0; c <= nfields; ++c) fb.lo[c] = field_lo[c];
   hipStream_t st = (hipStream_t)stream;
@@ -1423,9 +1822,9 @@ extern "C" int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t 
   k_field_keys<<<dim3((unsigned)cdiv(nrows, kFieldKeyRows), (unsigned)nfields), 256, 0, st>>>(
       ids, nrows, (int)nfields, fb, (uint32_t*)S.keys[1]);
   k_field_sort<<<(unsigned)nfields, kFieldThreads, 0, st>>>((const uint32_t*)S.keys[1], nrows, (int)nfields, fb,
-                                                            (uint32_t*)S.keys[0], sv, S.hist, S.d_tot + 2);
+                                                            (uint32_t*)S.keys[0], sv, S.fcnt, S.d_tot + 2);
   k_field_apply<<<(unsigned)nfields, kFieldThreads, 0, st>>>((const uint32_t*)S.keys[0], sv, nrows, (int)nfields, fb,
-                                                             S.hist, S.d_tot, n_unique, uniq, S.seg_start,
+                                                             S.fcnt, S.d_tot, n_unique, uniq, S.seg_start,
                                                              S.seg_occ0, inverse, S.chunk_off, S.chunk_seg,
                                                              S.hot_list);
   return launch_status();
@@ -1468,7 +1867,7 @@ static int segment_sum_plan(const float* grad, int64_t n, int64_t D, int key_bit
 template <int VPL>
 static void seg_final_with(const float* grad, const int32_t* sv, DedupScratch& S, const int64_t* perm, int64_t n,
                            float* out, int64_t nrows, const DirLstepsHits& first, int64_t nb1, hipStream_t st) {
-  const int64_t hb = n / kHotLen + 1;
+  const int64_t hb = hot_max(n);
   const SegFinalWpr<VPL, 0> f{grad, sv, S.seg_start, S.seg_occ0, perm, S.chunk_off, S.parts, S.d_tot, 0,
                               S.hot_list, S.d_tot + 2, hb, out, nrows, AdamScalars{}};
   launch2(first, nb1, f, hb + cdiv(n, 4 * kSegPerWave), st);

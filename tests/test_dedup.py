@@ -291,6 +291,63 @@ def test_gpu_segment_lengths_at_every_boundary(dev, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('n', [1, 17, 3072, 3073, 20_000])
+@pytest.mark.parametrize('D', [4, 12, 16, 24, 48, 100, 192, 320])
+def test_gpu_segment_lengths_in_chunk_layout(dev, D, n):
+    """Widths whose rows move in 16-byte chunks (a multiple of 4 other than 64, 128, 256, 512; each number of lanes per
+    row and two chunks per lane), both summation orders, with ids on each boundary of the work split: runs of 10,
+    the lanes' 4 to 64 occurrence indices, windows of 16, the hot limits (64 windowed, 240 sorted), a hot id that fills
+    the staging area several times.  Sums bitwise ATen's on this GPU and the oracle's, the fused Adam the oracle's."""
+    from elara_amd.dedup import adam_dedup, embedding_dense_backward
+    print(f'[gpu-test] chunk layout D={D} n={n}', flush=True)
+    rng = np.random.default_rng(n + D)
+    lens = [1, 2, 3, 4, 5, 8, 9, 10, 11, 15, 16, 17, 20, 21, 32, 33, 60, 61, 64, 65, 66, 240, 241, 600]
+    lens = lens + [1100] if n > 3072 else lens
+    ids = np.concatenate([np.full(L, 10 + 7 * k) for k, L in enumerate(lens)])[:n]
+    ids = np.concatenate([ids, 1000 + np.arange(n - ids.size)])
+    ids = ids[rng.permutation(n)].astype(np.int64)
+    U = 1000 + n
+    g = (rng.standard_normal((n, D)) * np.exp2(rng.integers(-12, 12, (n, 1)))).astype(np.float32)
+    gd, idd = torch.from_numpy(g).to(dev), torch.from_numpy(ids).to(dev)
+    want = full_sums(ids, g, U)
+    got = embedding_dense_backward(gd, idd, U)
+    aten = torch.ops.aten.embedding_dense_backward(gd, idd, U, -1, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got.cpu().numpy()), bits(want))
+    assert np.array_equal(bits(aten.cpu().numpy()), bits(want))
+    state = np.zeros((U, 3, D), np.float32)
+    state[:, 0] = (rng.standard_normal((U, D)) * 0.05).astype(np.float32)
+    gpu = torch.from_numpy(state).to(dev)
+    u, s, _ = O.segment_sum(ids, g)
+    O.cpu_adam(state, u, s, O.adam_scalars(*HP, 3), 8)
+    adam_dedup(gpu, idd, gd, *HP, 3)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(gpu.cpu().numpy()), bits(state))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [(1 << 22) + 1, 9_000, 530_000])
+def test_gpu_sort_and_segments_at_their_limits(dev, n):
+    """The sort with its digit counts added up in the scatter (up to 128 tiles of 4,096) and from a scan launch, the
+    segment offsets from the blocks and (above 2,048 tiles) from a scan launch, an id that spans many tiles and ids
+    whose segment ends in a later tile: unique equals torch.unique and the sums equal ATen's."""
+    from elara_amd.dedup import embedding_dense_backward, unique
+    print(f'[gpu-test] sort and segments n={n}', flush=True)
+    U, D = n // 3 + 2, 8
+    gen = torch.Generator(dev).manual_seed(n)
+    ids = torch.randint(0, U, (n,), device=dev, generator=gen)
+    ids[torch.rand(n, device=dev, generator=gen) < 0.3] = U // 2
+    ids[torch.rand(n, device=dev, generator=gen) < 0.01] = U - 1
+    g = torch.randn(n, D, device=dev, generator=gen)
+    u, inv = unique(ids, bound=U)
+    tu, tinv = torch.unique(ids, return_inverse=True)
+    assert torch.equal(u, tu) and torch.equal(inv, tinv)
+    want = torch.ops.aten.embedding_dense_backward(g, ids, U, -1, False)
+    got = embedding_dense_backward(g, ids, U)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.gpu
 def test_gpu_aten_golden_cases(dev):
     """The HIP sum reproduces the committed ATen vectors (both paths, -0.0 ids, hot ids)."""
     from elara_amd.dedup import embedding_dense_backward
