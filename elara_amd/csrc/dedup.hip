@@ -585,12 +585,95 @@ struct FieldBounds {
   int64_t lo[kFieldMax + 1];
 };
 
-// Passes and digit width for keys in [0, span]: ceil(bits / kFieldDigit) passes of equal width.
+// Passes and digit width for keys of `bits` bits, or in [0, span]: ceil(bits / kFieldDigit) passes of equal width.
+__host__ __device__ __forceinline__ void digits_for(int bits, int& passes, int& rb) {
+  passes = (bits + kFieldDigit - 1) / kFieldDigit;
+  rb = (bits + passes - 1) / passes;
+}
 __device__ __forceinline__ void field_digits(int64_t span, int& passes, int& rb) {
   int bits = 1;
   while (bits < 31 && (int64_t(1) << bits) <= span) ++bits;
-  passes = (bits + kFieldDigit - 1) / kFieldDigit;
-  rb = (bits + passes - 1) / passes;
+  digits_for(bits, passes, rb);
+}
+
+// A stable sort of at most kFieldThreads * ITEMS keys by one block in LDS: thread t of wave w holds items
+// (w * ITEMS + r) * 64 + lane in kk[r] and ends with the sorted keys of those positions; the result is each sorted
+// key's item index.  LSD passes of rb-bit digits, each key ranked as in k_radix_scatter (ballots, a running count per
+// wave, a scan over the waves).  s.lk holds the sorted keys too.
+template <typename Key, int ITEMS>
+struct BlockSort {
+  static constexpr int N = kFieldThreads * ITEMS, BINS = 1 << kFieldDigit, NW = kFieldThreads / 64;
+  Key lk[N + 1];
+  uint16_t lv[2][N];      // pass p writes lv[p & 1]
+  uint16_t wc[NW][BINS];  // per wave: running count of digit d, then the count in earlier waves
+  int lbase[BINS];
+  int wtot[NW];
+};
+
+template <typename Key, int ITEMS>
+__device__ __forceinline__ const uint16_t* block_sort(BlockSort<Key, ITEMS>& s, Key (&kk)[ITEMS], int n, int passes,
+                                                      int rb) {
+  constexpr int NW = kFieldThreads / 64, WSPAN = ITEMS * 64;
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  const int nbins = 1 << rb;
+  const uint32_t mask = (uint32_t)nbins - 1u;
+  for (int p = 0; p < passes; ++p) {
+    const int shift = p * rb;
+    const uint16_t* vsrc = s.lv[(p + 1) & 1];
+    uint16_t* vdst = s.lv[p & 1];
+    if (t < nbins)
+#pragma unroll
+      for (int q = 0; q < NW; ++q) s.wc[q][t] = 0;
+    __syncthreads();
+    int rk[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      const bool valid = w * WSPAN + r * 64 + lane < n;
+      const uint32_t d = (uint32_t)(kk[r] >> shift) & mask;
+      uint64_t m = __ballot(valid);
+      for (int b = 0; b < rb; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const uint64_t bal = __ballot(bit);
+        m &= bit ? bal : ~bal;
+      }
+      const int lr = __popcll(m & lanemask_lt());
+      // one wave's LDS accesses take effect in program order: every lane reads the count before the lowest lane of
+      // its digit group adds the group's size
+      const int before = valid ? (int)s.wc[w][d] : 0;
+      rk[r] = valid ? before + lr : -1;
+      if (valid && lr == 0) s.wc[w][d] = (uint16_t)(before + __popcll(m));
+    }
+    __syncthreads();
+    int run = 0;
+    if (t < nbins)
+#pragma unroll
+      for (int q = 0; q < NW; ++q) {
+        const int x = s.wc[q][t];
+        s.wc[q][t] = (uint16_t)run;
+        run += x;
+      }
+    {
+      int v[1] = {run}, ex[1], tot[1];
+      block_excl_scan<kFieldThreads, 1>(v, ex, tot);
+      if (t < nbins) s.lbase[t] = ex[0];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+      if (rk[r] >= 0) {
+        const int j = w * WSPAN + r * 64 + lane;
+        const uint32_t d = (uint32_t)(kk[r] >> shift) & mask;
+        const int lp = s.lbase[d] + s.wc[w][d] + rk[r];
+        s.lk[lp] = kk[r];
+        vdst[lp] = p == 0 ? (uint16_t)j : vsrc[j];
+      }
+    __syncthreads();
+    // (unconditional: items past n hold anything, and a load under a condition per item makes the compiler keep the
+    // array as one 16-register value and spill it around every branch)
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) kk[r] = s.lk[w * WSPAN + r * 64 + lane];
+  }
+  return s.lv[(passes - 1) & 1];
 }
 
 // Head flags of the sorted column in lk (bit r: this thread's item r, position w * kFieldItems * 64 + r * 64 +
@@ -657,97 +740,33 @@ __global__ __launch_bounds__(kFieldThreads) void k_field_sort(const uint32_t* __
                                                               int nf, FieldBounds fb, uint32_t* __restrict__ skeys,
                                                               int32_t* __restrict__ svals, int64_t* __restrict__ cnt,
                                                               int64_t* __restrict__ d_hot) {
-  constexpr int NW = kFieldThreads / 64, WSPAN = kFieldItems * 64, BINS = 1 << kFieldDigit;
-  __shared__ uint32_t lk[kFieldRows + 1];   // the column by digit; at the end the head positions (U + 1 of them)
-  __shared__ uint16_t lv[2][kFieldRows];    // sample index of each key: pass p writes lv[p & 1]
-  __shared__ uint16_t wc[NW][BINS];         // per wave: running count of digit d, then the count in earlier waves
-  __shared__ int lbase[BINS];
-  __shared__ int wtot[NW];
+  __shared__ BlockSort<uint32_t, kFieldItems> s;   // at the end its keys hold the head positions (U + 1 of them)
   const int c = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
   const int n = (int)nrows;
   const int64_t R = fb.lo[c + 1] - fb.lo[c];
   int passes, rb;
   field_digits(R, passes, rb);
-  const int nbins = 1 << rb;
-  const uint32_t mask = (uint32_t)nbins - 1u;
   if (c == 0 && t == 0) *d_hot = 0;
   uint32_t kk[kFieldItems];
 #pragma unroll
   for (int r = 0; r < kFieldItems; ++r) {
-    const int j = w * WSPAN + r * 64 + lane;
-    kk[r] = j < n ? keys[(int64_t)c * nrows + j] : 0u;
+    const int j = (w * kFieldItems + r) * 64 + lane;
+    kk[r] = keys[(int64_t)c * nrows + (j < n ? j : 0)];
   }
-  for (int p = 0; p < passes; ++p) {
-    const int shift = p * rb;
-    const uint16_t* vsrc = lv[(p + 1) & 1];
-    uint16_t* vdst = lv[p & 1];
-    if (t < nbins)
-#pragma unroll
-      for (int q = 0; q < NW; ++q) wc[q][t] = 0;
-    __syncthreads();
-    int rk[kFieldItems];
-#pragma unroll
-    for (int r = 0; r < kFieldItems; ++r) {
-      const bool valid = w * WSPAN + r * 64 + lane < n;
-      const uint32_t d = (kk[r] >> shift) & mask;
-      uint64_t m = __ballot(valid);
-      for (int b = 0; b < rb; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t bal = __ballot(bit);
-        m &= bit ? bal : ~bal;
-      }
-      const int lr = __popcll(m & lanemask_lt());
-      // one wave's LDS accesses take effect in program order: every lane reads the count before the lowest lane of
-      // its digit group adds the group's size
-      const int before = valid ? (int)wc[w][d] : 0;
-      rk[r] = valid ? before + lr : -1;
-      if (valid && lr == 0) wc[w][d] = (uint16_t)(before + __popcll(m));
-    }
-    __syncthreads();
-    int run = 0;
-    if (t < nbins)
-#pragma unroll
-      for (int q = 0; q < NW; ++q) {
-        const int x = wc[q][t];
-        wc[q][t] = (uint16_t)run;
-        run += x;
-      }
-    {
-      int v[1] = {run}, ex[1], tot[1];
-      block_excl_scan<kFieldThreads, 1>(v, ex, tot);
-      if (t < nbins) lbase[t] = ex[0];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kFieldItems; ++r)
-      if (rk[r] >= 0) {
-        const int j = w * WSPAN + r * 64 + lane;
-        const uint32_t d = (kk[r] >> shift) & mask;
-        const int lp = lbase[d] + wc[w][d] + rk[r];
-        lk[lp] = kk[r];
-        vdst[lp] = p == 0 ? (uint16_t)j : vsrc[j];
-      }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kFieldItems; ++r) {
-      const int j = w * WSPAN + r * 64 + lane;
-      if (j < n) kk[r] = lk[j];
-    }
-  }
-  const uint16_t* vfin = lv[(passes - 1) & 1];
+  const uint16_t* vfin = block_sort<uint32_t, kFieldItems>(s, kk, n, passes, rb);
   const int64_t out0 = (int64_t)c * nrows;
 #pragma unroll
   for (int r = 0; r < kFieldItems; ++r) {
-    const int j = w * WSPAN + r * 64 + lane;
+    const int j = (w * kFieldItems + r) * 64 + lane;
     if (j < n) {
       skeys[out0 + j] = kk[r];
       svals[out0 + j] = (int32_t)vfin[j] * nf + c;
     }
   }
   int wcount;
-  const uint32_t hm = field_heads(lk, n, wcount);
-  int* hpos = reinterpret_cast<int*>(lk);
-  const int U = field_head_positions(hm, wcount, n, wtot, hpos);
+  const uint32_t hm = field_heads(s.lk, n, wcount);
+  int* hpos = reinterpret_cast<int*>(s.lk);
+  const int U = field_head_positions(hm, wcount, n, s.wtot, hpos);
   int e = 0;
   for (int u = t; u < U; u += kFieldThreads) e += part_chunks(hpos[u + 1] - hpos[u]);
   int v[1] = {e}, ex[1], tot[1];
@@ -853,6 +872,98 @@ __global__ __launch_bounds__(kFieldThreads) void k_field_apply(const uint32_t* _
     if (n_unique) *n_unique = Ut;
     seg_start[Ut] = out0 + n;
     d_tot[1] = before;
+  }
+}
+
+// The whole dedup plan of at most kFieldThreads * ITEMS ids by one block: the sort in LDS, the segment heads from
+// ballots, the inverse, the hot segments and the partial-chunk plan -- what the radix passes, k_seg_count and
+// k_seg_apply leave, in one launch.  SMALLPLAN
+constexpr int kSmallItems = 4;
+constexpr int64_t kSmallPlan = kFieldThreads * kSmallItems;
+template <typename Key, int ITEMS>
+__global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __restrict__ ids, int n, int passes, int rb,
+                                                              int32_t* __restrict__ svals, int64_t* __restrict__ d_tot,
+                                                              int64_t* __restrict__ n_unique,
+                                                              int64_t* __restrict__ uniq,
+                                                              int64_t* __restrict__ seg_start,
+                                                              int32_t* __restrict__ seg_occ0,
+                                                              int64_t* __restrict__ inverse,
+                                                              int32_t* __restrict__ chunk_off,
+                                                              int32_t* __restrict__ chunk_seg,
+                                                              int32_t* __restrict__ hot_list, int hot_len) {
+  constexpr int NW = kFieldThreads / 64;
+  __shared__ BlockSort<Key, ITEMS> s;
+  __shared__ int wfirst[NW], ecnt, hcnt;
+  const int t = threadIdx.x, w = block_wave(), lane = t & 63;
+  Key kk[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = (w * ITEMS + r) * 64 + lane;
+    kk[r] = (Key)ids[j < n ? j : 0];
+  }
+  if (t == 0) ecnt = hcnt = 0;
+  const uint16_t* vfin = block_sort<Key, ITEMS>(s, kk, n, passes, rb);
+  uint64_t hm[ITEMS];
+  int c = 0, first = n;
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    const int j = (w * ITEMS + r) * 64 + lane;
+    hm[r] = __builtin_amdgcn_ballot_w64(j < n && (j == 0 || s.lk[j > 0 ? j - 1 : 0] != kk[r]));
+    c += __builtin_popcountll(hm[r]);
+    if (hm[r]) first = (w * ITEMS + r) * 64 + __builtin_ctzll(hm[r]);
+  }
+  if (lane == 0) {
+    s.wtot[w] = c;
+    wfirst[w] = first;
+  }
+  __syncthreads();
+  int run = 0, U = 0, nxt = n;
+#pragma unroll
+  for (int q = 0; q < NW; ++q) {
+    run += q < w ? s.wtot[q] : 0;
+    U += s.wtot[q];
+  }
+#pragma unroll
+  for (int q = NW - 1; q >= 0; --q)
+    if (q > w && wfirst[q] < n) nxt = wfirst[q];
+  int end = run + c;
+#pragma unroll
+  for (int r = ITEMS - 1; r >= 0; --r) {
+    const int j = (w * ITEMS + r) * 64 + lane;
+    const uint64_t m = hm[r];
+    const bool head = (m >> lane) & 1;
+    const int u0 = end - __builtin_popcountll(m), u = u0 + __builtin_popcountll(m & lanemask_lt()) + (head ? 0 : -1);
+    end = u0;
+    if (j < n) {
+      const int o = vfin[j];
+      svals[j] = o;
+      if (inverse) inverse[o] = u;
+      if (head) {
+        uniq[u] = (int64_t)kk[r];
+        seg_start[u] = j;
+        seg_occ0[u] = o;
+        if (hot_list) {
+          const uint64_t up = lane == 63 ? 0ull : m >> (lane + 1);
+          const int L = up ? (int)__builtin_ctzll(up) + 1 : nxt - j;
+          const int e = chunk_off ? part_chunks(L) : 0;
+          if (e > 0) {
+            const int off = atomicAdd(&ecnt, e);
+            chunk_off[u] = off;
+            for (int k = 0; k < e; ++k) chunk_seg[off + k] = u;
+          }
+          if (L > hot_len) hot_list[atomicAdd(&hcnt, 1)] = u;
+        }
+      }
+    }
+    if (m) nxt = (w * ITEMS + r) * 64 + __builtin_ctzll(m);
+  }
+  __syncthreads();
+  if (t == 0) {
+    d_tot[0] = U;
+    d_tot[1] = ecnt;
+    d_tot[2] = hcnt;
+    if (n_unique) *n_unique = U;
+    seg_start[U] = n;
   }
 }
 
@@ -1601,9 +1712,23 @@ static void seg_plan(const Key* sk, const int32_t* sv, int64_t n, DedupScratch& 
 template <typename Key>
 static int dedup_core(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, int64_t* uniq_out,
                       int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
+  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
+  if (n <= kSmallPlan) {
+    int passes, rb;
+    digits_for(key_bits, passes, rb);
+    const int cur = (sort_passes<Key>(key_bits) - 1) % 2;   // where the radix passes would leave the positions
+    auto go = [&](auto kern) {
+      kern<<<1, kFieldThreads, 0, st>>>(ids, (int)n, passes, rb, S.vals[cur], S.d_tot, n_unique, uniq, S.seg_start,
+                                        S.seg_occ0, inverse, win_shift_for(n) ? nullptr : S.chunk_off, S.chunk_seg,
+                                        sums ? S.hot_list : nullptr, (int)(win_shift_for(n) ? kWinHot : kHotLen));
+    };
+    if (n <= kFieldThreads) go(k_small_plan<Key, 1>);
+    else if (n <= 2 * kFieldThreads) go(k_small_plan<Key, 2>);
+    else go(k_small_plan<Key, kSmallItems>);
+    return cur;
+  }
   const int cur = radix_sort<Key>(ids, n, key_bits, S, st);
   const Key* sk = (const Key*)S.keys[cur];
-  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
   if (seg_items_for(n) == kSegItemsBig)
     seg_plan<Key, kSegItemsBig>(sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
   else
