@@ -314,10 +314,32 @@ constexpr int kSegWaves = kSegBlock / 64;
 __device__ __forceinline__ int lane_value(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
 __device__ __forceinline__ int block_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// What the sorted keys stand for: ids (PlainKeys), or one field's column after the other, each key an offset in its
+// field's rows (FieldKeys, elr_dedup_plan_fields), where a column's first position is a head whatever its key.
+struct PlainKeys {
+  template <typename Key>
+  __device__ __forceinline__ int64_t id(Key k, int64_t) const { return (int64_t)k; }
+  __device__ __forceinline__ bool starts(int64_t i) const { return i == 0; }
+};
+constexpr int kFieldMax = 128;   // fields per batch (the bounds travel as a kernel argument)
+struct FieldBounds {
+  int64_t lo[kFieldMax + 1];
+};
+struct FieldKeys {
+  FieldBounds fb;
+  uint32_t nrows;   // positions per column
+  __device__ __forceinline__ int64_t id(uint32_t k, int64_t i) const {   // -1: an id outside its field's rows
+    const uint32_t c = (uint32_t)i / nrows;
+    const int64_t lo = fb.lo[c], R = fb.lo[c + 1] - lo;
+    return (int64_t)k == R ? -1 : lo + (int64_t)k;
+  }
+  __device__ __forceinline__ bool starts(int64_t i) const { return (uint32_t)i % nrows == 0; }
+};
+
 // The wave's keys of sorted positions p0 + r * 64 + lane, and each round's head mask.
-template <typename Key, int ITEMS>
-__device__ __forceinline__ void seg_heads(const Key* __restrict__ sk, int64_t p0, int64_t n, Key (&kk)[ITEMS],
-                                          uint64_t (&hm)[ITEMS]) {
+template <typename Key, int ITEMS, class Keys>
+__device__ __forceinline__ void seg_heads(const Keys& keys, const Key* __restrict__ sk, int64_t p0, int64_t n,
+                                          Key (&kk)[ITEMS], uint64_t (&hm)[ITEMS]) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
@@ -330,15 +352,15 @@ __device__ __forceinline__ void seg_heads(const Key* __restrict__ sk, int64_t p0
     const int64_t i = p0 + r * 64 + lane;
     Key left = __shfl_up(kk[r], 1, 64);
     if (lane == 0) left = prev;
-    hm[r] = __builtin_amdgcn_ballot_w64(i < n && (i == 0 || kk[r] != left));
+    hm[r] = __builtin_amdgcn_ballot_w64(i < n && (keys.starts(i) || kk[r] != left));
     prev = __shfl(kk[r], 63, 64);
   }
 }
 
 // Segment heads: per-block head counts and first head position (n when the tile has none).  Also clears the counts
 // that k_seg_apply's chunk plan adds to.
-template <typename Key, int ITEMS>
-__global__ __launch_bounds__(kSegBlock) void k_seg_count(const Key* __restrict__ sk, int64_t n,
+template <typename Key, int ITEMS, class Keys>
+__global__ __launch_bounds__(kSegBlock) void k_seg_count(Keys keys, const Key* __restrict__ sk, int64_t n,
                                                          int64_t* __restrict__ bsum, int32_t* __restrict__ bfirst,
                                                          int64_t* __restrict__ d_E, int64_t* __restrict__ d_hot) {
   __shared__ int wcnt[kSegWaves];
@@ -347,7 +369,7 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_count(const Key* __restrict__
   const int64_t p0 = ((int64_t)blockIdx.x * kSegWaves + w) * (64 * ITEMS);
   Key kk[ITEMS];
   uint64_t hm[ITEMS];
-  seg_heads<Key, ITEMS>(sk, p0, n, kk, hm);
+  seg_heads<Key, ITEMS, Keys>(keys, sk, p0, n, kk, hm);
   int c = 0;
   int first = (int)n;
 #pragma unroll
@@ -416,9 +438,9 @@ __device__ __forceinline__ int part_chunks(int64_t L) {
 // add, so their order over the segments is not fixed; no sum depends on it (each group sum has its own parts row).
 // One launch in place of three (heads with a block scan per round, chunk counts, chunk plan): 28 us against 20 + 8 +
 // 20 and two scan launches of 4.5 at config C3's 3.4M positions, 10 against 18 + 8 + 21 at C5's 426k.
-template <typename Key, int ITEMS>
-__global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__ sk, const int32_t* __restrict__ sv,
-                                                         int64_t n, const int64_t* __restrict__ bcnt, int scanned,
+template <typename Key, int ITEMS, class Keys>
+__global__ __launch_bounds__(kSegBlock) void k_seg_apply(Keys keys, const Key* __restrict__ sk,
+                                                         const int32_t* __restrict__ sv, int64_t n, const int64_t* __restrict__ bcnt, int scanned,
                                                          const int32_t* __restrict__ bfirst,
                                                          int64_t* __restrict__ d_U, int64_t* __restrict__ n_unique,
                                                          int64_t* __restrict__ uniq, int64_t* __restrict__ seg_start,
@@ -441,7 +463,7 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__
     const int64_t i = p0 + r * 64 + lane;
     vv[r] = i < n ? sv[i] : -1;
   }
-  seg_heads<Key, ITEMS>(sk, p0, n, kk, hm);
+  seg_heads<Key, ITEMS, Keys>(keys, sk, p0, n, kk, hm);
   // the first head past this tile (n: none)
   int nxt = (int)n;
   for (int64_t b0 = (int64_t)blockIdx.x + 1; b0 < nblk; b0 += 64) {
@@ -493,7 +515,7 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__
     const int64_t u = u0 + __builtin_popcountll(m & lanemask_lt()) + (head ? 0 : -1);
     after[r] = nxt;
     if (head) {
-      uniq[u] = (int64_t)kk[r];
+      uniq[u] = keys.id(kk[r], i);
       seg_start[u] = i;
       seg_occ0[u] = vv[r];
     }
@@ -568,22 +590,17 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(const Key* __restrict__
 // whole batch is field 0's column sorted stably, then field 1's, and so on (within a column, sample order is
 // occurrence order).  One block per field sorts its column of at most kFieldRows ids in LDS: LSD passes of at most
 // kFieldDigit bits over the id's offset in its field, each key ranked as in k_radix_scatter (ballots, a running
-// count per wave, a scan over the waves), the column re-read from LDS after each pass.  The plan is then the
-// general path's, bit for bit, in three launches (k_field_keys, the columns' keys; k_field_sort; k_field_apply, which
-// adds the earlier fields' segment and chunk counts) instead of three per radix pass and four for the segments and
-// chunks.  An id outside
-// its field's rows takes the key R_c (the field's row count), sorts after the field's ids and comes out as -1 in
-// uniq: a row out of range for the caller.
+// count per wave, a scan over the waves), the column re-read from LDS after each pass.  The segments and chunks then
+// come from the general path's two launches (k_seg_count, k_seg_apply with FieldKeys), so the plan is the general
+// path's, bit for bit, in four launches.  A thread holds as many keys as the column needs (1 to 16).  (The
+// segments by one block per field, as the sort's, took 28 us of a 26-column batch of 426k; the two launches over
+// the whole GPU FIELDSEG.)  An id outside its field's rows takes the key R_c (the field's row count), sorts after the
+// field's ids and comes out as -1 in uniq: a row out of range for the caller.
 constexpr int kFieldThreads = 1024;
 constexpr int kFieldItems = 16;
 constexpr int64_t kFieldRows = (int64_t)kFieldThreads * kFieldItems;   // samples per batch: the row index is 16-bit
 constexpr int kFieldDigit = 9;
-constexpr int kFieldMax = 128;                      // fields per batch (the bounds travel as a kernel argument)
 constexpr int64_t kFieldSpanMax = (int64_t(1) << 31) - 2;   // rows per field: keys 0 .. R_c fit in 31 bits
-
-struct FieldBounds {
-  int64_t lo[kFieldMax + 1];
-};
 
 // Passes and digit width for keys of `bits` bits, or in [0, span]: ceil(bits / kFieldDigit) passes of equal width.
 __host__ __device__ __forceinline__ void digits_for(int bits, int& passes, int& rb) {
@@ -676,47 +693,6 @@ __device__ __forceinline__ const uint16_t* block_sort(BlockSort<Key, ITEMS>& s, 
   return s.lv[(passes - 1) & 1];
 }
 
-// Head flags of the sorted column in lk (bit r: this thread's item r, position w * kFieldItems * 64 + r * 64 +
-// lane) and this wave's head count.
-__device__ __forceinline__ uint32_t field_heads(const uint32_t* lk, int n, int& wcount) {
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint32_t hm = 0;
-  wcount = 0;
-#pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const int j = w * kFieldItems * 64 + r * 64 + lane;
-    const bool h = j < n && (j == 0 || lk[j - 1] != lk[j]);
-    hm |= h ? 1u << r : 0u;
-    wcount += __popcll(__ballot(h));
-  }
-  return hm;
-}
-
-// Positions of the column's segment heads, hpos[u] for u < U, and hpos[U] = n, from the head flags; returns U.
-// Synchronises the block before writing (hpos may share LDS with what the head test read) and after.
-__device__ __forceinline__ int field_head_positions(uint32_t hm, int wcount, int n, int* wtot, int* hpos) {
-  constexpr int NW = kFieldThreads / 64;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) wtot[w] = wcount;
-  __syncthreads();
-  int U = 0, run = 0;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    U += wtot[q];
-    run += q < w ? wtot[q] : 0;
-  }
-#pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const bool h = (hm >> r) & 1u;
-    const uint64_t bal = __ballot(h);
-    if (h) hpos[run + __popcll(bal & lanemask_lt())] = w * kFieldItems * 64 + r * 64 + lane;
-    run += __popcll(bal);
-  }
-  if (threadIdx.x == 0) hpos[U] = n;
-  __syncthreads();
-  return U;
-}
-
 // Each field's ids as offsets in its field (the key R_c for an id outside it), field after field: keys[c * nrows + j].
 // One block per field and kFieldKeyRows samples, so that the gather of a column (each wave's 64 loads touch 64
 // different cache lines) is spread over the whole GPU instead of being done by the field's sorting block alone.
@@ -736,149 +712,38 @@ __global__ __launch_bounds__(256) void k_field_keys(const int64_t* __restrict__ 
   }
 }
 
+// Each field's column sorted by one block (ITEMS keys per thread): skeys, and the occurrence index of each position.
+template <int ITEMS>
 __global__ __launch_bounds__(kFieldThreads) void k_field_sort(const uint32_t* __restrict__ keys, int64_t nrows,
                                                               int nf, FieldBounds fb, uint32_t* __restrict__ skeys,
-                                                              int32_t* __restrict__ svals, int64_t* __restrict__ cnt,
-                                                              int64_t* __restrict__ d_hot) {
-  __shared__ BlockSort<uint32_t, kFieldItems> s;   // at the end its keys hold the head positions (U + 1 of them)
-  const int c = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
+                                                              int32_t* __restrict__ svals) {
+  __shared__ BlockSort<uint32_t, ITEMS> s;
+  const int c = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = (int)nrows;
-  const int64_t R = fb.lo[c + 1] - fb.lo[c];
   int passes, rb;
-  field_digits(R, passes, rb);
-  if (c == 0 && t == 0) *d_hot = 0;
-  uint32_t kk[kFieldItems];
+  field_digits(fb.lo[c + 1] - fb.lo[c], passes, rb);
+  uint32_t kk[ITEMS];
 #pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const int j = (w * kFieldItems + r) * 64 + lane;
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = (w * ITEMS + r) * 64 + lane;
     kk[r] = keys[(int64_t)c * nrows + (j < n ? j : 0)];
   }
-  const uint16_t* vfin = block_sort<uint32_t, kFieldItems>(s, kk, n, passes, rb);
+  const uint16_t* vfin = block_sort<uint32_t, ITEMS>(s, kk, n, passes, rb);
   const int64_t out0 = (int64_t)c * nrows;
 #pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const int j = (w * kFieldItems + r) * 64 + lane;
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = (w * ITEMS + r) * 64 + lane;
     if (j < n) {
       skeys[out0 + j] = kk[r];
       svals[out0 + j] = (int32_t)vfin[j] * nf + c;
     }
-  }
-  int wcount;
-  const uint32_t hm = field_heads(s.lk, n, wcount);
-  int* hpos = reinterpret_cast<int*>(s.lk);
-  const int U = field_head_positions(hm, wcount, n, s.wtot, hpos);
-  int e = 0;
-  for (int u = t; u < U; u += kFieldThreads) e += part_chunks(hpos[u + 1] - hpos[u]);
-  int v[1] = {e}, ex[1], tot[1];
-  block_excl_scan<kFieldThreads, 1>(v, ex, tot);
-  if (t == 0) {
-    cnt[2 * c] = U;
-    cnt[2 * c + 1] = tot[0];
-  }
-}
-
-// Field c's unique ids, segment starts, first occurrences, inverse and chunk plan, offset by the earlier fields'
-// segment and chunk counts (cnt, from k_field_sort).  The last field's block stores U, E and seg_start[U] = n.
-__global__ __launch_bounds__(kFieldThreads) void k_field_apply(const uint32_t* __restrict__ skeys,
-                                                               const int32_t* __restrict__ svals, int64_t nrows,
-                                                               int nf, FieldBounds fb, const int64_t* __restrict__ cnt,
-                                                               int64_t* __restrict__ d_tot,
-                                                               int64_t* __restrict__ n_unique,
-                                                               int64_t* __restrict__ uniq,
-                                                               int64_t* __restrict__ seg_start,
-                                                               int32_t* __restrict__ seg_occ0,
-                                                               int64_t* __restrict__ inverse,
-                                                               int32_t* __restrict__ chunk_off,
-                                                               int32_t* __restrict__ chunk_seg,
-                                                               int32_t* __restrict__ hot_list) {
-  constexpr int NW = kFieldThreads / 64, WSPAN = kFieldItems * 64;
-  __shared__ uint32_t lk[kFieldRows];
-  __shared__ int hpos[kFieldRows + 1];
-  __shared__ int wtot[NW];
-  __shared__ int64_t pre[2][NW];
-  const int c = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int n = (int)nrows;
-  const int64_t lo = fb.lo[c], R = fb.lo[c + 1] - lo, out0 = (int64_t)c * nrows;
-  {
-    // segments and chunks of the earlier fields (nf <= kFieldMax <= kFieldThreads)
-    int64_t a = t < c ? cnt[2 * t] : 0, b = t < c ? cnt[2 * t + 1] : 0;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-      a += __shfl_xor(a, d, 64);
-      b += __shfl_xor(b, d, 64);
-    }
-    if (lane == 0) {
-      pre[0][w] = a;
-      pre[1][w] = b;
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const int j = w * WSPAN + r * 64 + lane;
-    if (j < n) lk[j] = skeys[out0 + j];
-  }
-  __syncthreads();
-  int64_t su = 0, se = 0;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    su += pre[0][q];
-    se += pre[1][q];
-  }
-  int wcount;
-  const uint32_t hm = field_heads(lk, n, wcount);
-  const int U = field_head_positions(hm, wcount, n, wtot, hpos);
-  // every position's segment: heads at or before it, less one (this wave's earlier heads from the head flags)
-  int run = 0;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) run += q < w ? wtot[q] : 0;
-#pragma unroll
-  for (int r = 0; r < kFieldItems; ++r) {
-    const int j = w * WSPAN + r * 64 + lane;
-    const bool h = (hm >> r) & 1u;
-    const uint64_t bal = __ballot(h);
-    if (j < n) {
-      const int64_t gu = su + run + __popcll(bal & lanemask_lt()) + (h ? 0 : -1);
-      const int32_t o = svals[out0 + j];
-      if (h) {
-        const uint32_t k = lk[j];
-        uniq[gu] = (int64_t)k == R ? -1 : lo + (int64_t)k;
-        seg_start[gu] = out0 + j;
-        seg_occ0[gu] = o;
-      }
-      if (inverse) inverse[o] = gu;
-    }
-    run += __popcll(bal);
-  }
-  int64_t before = se;
-  for (int u0 = 0; u0 < U; u0 += kFieldThreads) {
-    const int u = u0 + t;
-    const int L = u < U ? hpos[u + 1] - hpos[u] : 0;
-    const int e = u < U ? part_chunks(L) : 0;
-    int v[1] = {e}, ex[1], tot[1];
-    block_excl_scan<kFieldThreads, 1>(v, ex, tot);
-    if (u < U) {
-      const int64_t off = before + ex[0];
-      const int32_t gu = (int32_t)(su + u);
-      chunk_off[gu] = (int32_t)off;
-      for (int k = 0; k < e; ++k) chunk_seg[off + k] = gu;
-      if (seg_hot(L)) hot_list[atomicAdd(reinterpret_cast<unsigned long long*>(d_tot + 2), 1ull)] = gu;
-    }
-    before += tot[0];
-    __syncthreads();   // block_excl_scan's LDS is reused by the next round
-  }
-  if (c == nf - 1 && t == 0) {
-    const int64_t Ut = su + U;
-    d_tot[0] = Ut;
-    if (n_unique) *n_unique = Ut;
-    seg_start[Ut] = out0 + n;
-    d_tot[1] = before;
   }
 }
 
 // The whole dedup plan of at most kFieldThreads * ITEMS ids by one block: the sort in LDS, the segment heads from
 // ballots, the inverse, the hot segments and the partial-chunk plan -- what the radix passes, k_seg_count and
 // k_seg_apply leave, in one launch.  SMALLPLAN
-constexpr int kSmallItems = 4;
+constexpr int kSmallItems = 8;
 constexpr int64_t kSmallPlan = kFieldThreads * kSmallItems;
 template <typename Key, int ITEMS>
 __global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __restrict__ ids, int n, int passes, int rb,
@@ -1581,7 +1446,6 @@ struct DedupScratch {
   int32_t* vals[2];
   int32_t* hist;      // [kRadixMaxBins * ntile] digit counts per sort tile (sort_tiles)
   int32_t* dtot;      // [kRadixMaxBins] digit totals
-  int64_t* fcnt;      // [2 * kFieldMax] segments and chunks of each field (elr_dedup_plan_fields)
   int64_t* bsum;      // [n / (kSegBlock * seg_items_for(n)) + 1] heads per segment tile
   int32_t* bfirst;    // the same count: each tile's first head
   int64_t* d_tot;     // [3]: U, E (partial chunks), hot segments
@@ -1594,10 +1458,9 @@ struct DedupScratch {
   int32_t* hot_list;  // [hot_max(n)] hot segments
 };
 
-// (the segment tiles' counts, at most kSegPerSort tiles per sort tile, fit beside the digit counts, and the fields'
-// counts beside the digit totals)
+// (the segment tiles' counts, at most kSegPerSort tiles per sort tile, fit beside the digit counts)
 constexpr int64_t kSegPerSort = kSortTile / (kSegBlock * kSegItemsSmall);
-static_assert(kSegPerSort * 12 <= kRadixMaxBins * 4 && 2 * kFieldMax * 8 <= kRadixMaxBins * 4, "shared scratch");
+static_assert(kSegPerSort * 12 <= kRadixMaxBins * 4, "shared scratch");
 
 inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void* base) {
   const int64_t ntile = sort_tiles(n), nblk = cdiv(n, kSegBlock * seg_items_for(n));
@@ -1614,12 +1477,11 @@ inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void
   s.keys[1] = take(n * 8);
   s.vals[0] = (int32_t*)take(n * 4);
   s.vals[1] = (int32_t*)take(n * 4);
-  // the digit counts, then the segment tiles' counts; the digit totals, then the fields' counts
+  // the digit counts, then the segment tiles' counts; the digit totals
   s.hist = (int32_t*)take(kRadixMaxBins * ntile * 8);
   s.bsum = (int64_t*)(s.hist + kRadixMaxBins * ntile);
   s.bfirst = (int32_t*)(s.bsum + nblk);
   s.dtot = (int32_t*)take(kRadixMaxBins * 8);
-  s.fcnt = (int64_t*)(s.dtot + kRadixMaxBins);
   o += al256(ntile * 8);   // unused: keeps the largest n of elr_adam_dedup_noalloc where it has been
   s.d_tot = (int64_t*)take(3 * 8);
   s.uniq = (int64_t*)take(n * 8);
@@ -1695,17 +1557,26 @@ static int radix_sort(const int64_t* ids, int64_t n, int key_bits, DedupScratch&
 
 // Segment heads (uniq / seg_start / inverse, U in d_tot[0]) of the sorted keys and, for segment sums (sums), the hot
 // segments and the partial-chunk plan (E in d_tot[1]; the windowed path has no partial chunks).
-template <typename Key, int ITEMS>
-static void seg_plan(const Key* sk, const int32_t* sv, int64_t n, DedupScratch& S, int64_t* uniq, int64_t* inverse,
+template <typename Key, int ITEMS, class Keys>
+static void seg_plan_items(const Keys& keys, const Key* sk, const int32_t* sv, int64_t n, DedupScratch& S, int64_t* uniq, int64_t* inverse,
                      int64_t* n_unique, bool sums, hipStream_t st) {
   const int64_t nblk = cdiv(n, kSegBlock * ITEMS);
   const int scanned = nblk > kFoldMaxBlocks;
-  k_seg_count<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(sk, n, S.bsum, S.bfirst, S.d_tot + 1, S.d_tot + 2);
+  k_seg_count<Key, ITEMS, Keys><<<(unsigned)nblk, kSegBlock, 0, st>>>(keys, sk, n, S.bsum, S.bfirst, S.d_tot + 1, S.d_tot + 2);
   if (scanned) k_scan_blocks<<<1, kScanBlock, 0, st>>>(S.bsum, nblk);
-  k_seg_apply<Key, ITEMS><<<(unsigned)nblk, kSegBlock, 0, st>>>(
-      sk, sv, n, S.bsum, scanned, S.bfirst, S.d_tot, n_unique, uniq, S.seg_start, S.seg_occ0, inverse,
+  k_seg_apply<Key, ITEMS, Keys><<<(unsigned)nblk, kSegBlock, 0, st>>>(
+      keys, sk, sv, n, S.bsum, scanned, S.bfirst, S.d_tot, n_unique, uniq, S.seg_start, S.seg_occ0, inverse,
       win_shift_for(n) ? nullptr : S.chunk_off, S.chunk_seg, sums ? S.hot_list : nullptr,
       (int)(win_shift_for(n) ? kWinHot : kHotLen), S.d_tot + 2, S.d_tot + 1);
+}
+
+template <typename Key, class Keys>
+static void seg_plan(const Keys& keys, const Key* sk, const int32_t* sv, int64_t n, DedupScratch& S, int64_t* uniq,
+                     int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
+  if (seg_items_for(n) == kSegItemsBig)
+    seg_plan_items<Key, kSegItemsBig, Keys>(keys, sk, sv, n, S, uniq, inverse, n_unique, sums, st);
+  else
+    seg_plan_items<Key, kSegItemsSmall, Keys>(keys, sk, sv, n, S, uniq, inverse, n_unique, sums, st);
 }
 
 // Sort, segment heads and partial-chunk plan; returns which buffer holds the sorted positions.
@@ -1724,15 +1595,13 @@ static int dedup_core(const int64_t* ids, int64_t n, int key_bits, DedupScratch&
     };
     if (n <= kFieldThreads) go(k_small_plan<Key, 1>);
     else if (n <= 2 * kFieldThreads) go(k_small_plan<Key, 2>);
+    else if (n <= 4 * kFieldThreads) go(k_small_plan<Key, 4>);
     else go(k_small_plan<Key, kSmallItems>);
     return cur;
   }
   const int cur = radix_sort<Key>(ids, n, key_bits, S, st);
   const Key* sk = (const Key*)S.keys[cur];
-  if (seg_items_for(n) == kSegItemsBig)
-    seg_plan<Key, kSegItemsBig>(sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
-  else
-    seg_plan<Key, kSegItemsSmall>(sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
+  seg_plan<Key>(PlainKeys{}, sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
   return cur;
 }
 
@@ -1946,12 +1815,18 @@ extern "C" int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t 
   int32_t* sv = S.vals[plan_result_buffer(key_bits)];
   k_field_keys<<<dim3((unsigned)cdiv(nrows, kFieldKeyRows), (unsigned)nfields), 256, 0, st>>>(
       ids, nrows, (int)nfields, fb, (uint32_t*)S.keys[1]);
-  k_field_sort<<<(unsigned)nfields, kFieldThreads, 0, st>>>((const uint32_t*)S.keys[1], nrows, (int)nfields, fb,
-                                                            (uint32_t*)S.keys[0], sv, S.fcnt, S.d_tot + 2);
-  k_field_apply<<<(unsigned)nfields, kFieldThreads, 0, st>>>((const uint32_t*)S.keys[0], sv, nrows, (int)nfields, fb,
-                                                             S.fcnt, S.d_tot, n_unique, uniq, S.seg_start,
-                                                             S.seg_occ0, inverse, S.chunk_off, S.chunk_seg,
-                                                             S.hot_list);
+  auto sort = [&](auto kern) {
+    kern<<<(unsigned)nfields, kFieldThreads, 0, st>>>((const uint32_t*)S.keys[1], nrows, (int)nfields, fb,
+                                                      (uint32_t*)S.keys[0], sv);
+  };
+  const int64_t per = cdiv(nrows, kFieldThreads);
+  if (per <= 1) sort(k_field_sort<1>);
+  else if (per <= 2) sort(k_field_sort<2>);
+  else if (per <= 4) sort(k_field_sort<4>);
+  else if (per <= 8) sort(k_field_sort<8>);
+  else sort(k_field_sort<kFieldItems>);
+  seg_plan<uint32_t>(FieldKeys{fb, (uint32_t)nrows}, (const uint32_t*)S.keys[0], sv, n, S, uniq, inverse, n_unique, true,
+                     st);
   return launch_status();
 }
 
