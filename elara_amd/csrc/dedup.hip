@@ -970,32 +970,7 @@ __global__ __launch_bounds__(256) void k_seg_final(const float* __restrict__ gra
   }
 }
 
-// Adam on a lane's chunks: adam_elem's operations with one range check for all of them (frag_adam).
-template <int NC>
-__device__ __forceinline__ void chunk_adam(ChunkFrag<NC>& w, ChunkFrag<NC>& m, ChunkFrag<NC>& v,
-                                           const ChunkFrag<NC>& g, const AdamScalars& s) {
-  RowFrag<4 * NC> fw, fm, fv, fg;
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      fw.v[4 * c + j] = w.v[c][j];
-      fm.v[4 * c + j] = m.v[c][j];
-      fv.v[4 * c + j] = v.v[c][j];
-      fg.v[4 * c + j] = g.v[c][j];
-    }
-  frag_adam<4 * NC>(fw, fm, fv, fg, s);
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      w.v[c][j] = fw.v[4 * c + j];
-      m.v[c][j] = fm.v[4 * c + j];
-      v.v[c][j] = fv.v[4 * c + j];
-    }
-}
-
-// The final sums (and Adam, MODE 1) in the chunk layout (elr_seg_dev.h): LPR lanes per segment, 64 / LPR segments per
+// The final sums (and Adam, MODE 1) in the chunk layout (elr_rowio.h): LPR lanes per segment, 64 / LPR segments per
 // wave, WIN: ATen's windowed order.  A one-occurrence segment, the common case, costs two dependent round trips (its
 // metadata; its gradient row and state), and a longer one two more per kSubRows occurrences.  The first hot_blocks
 // blocks take the segments of hot_list, one each at a time: the whole block loads the run sums (windowed: the
@@ -1026,20 +1001,20 @@ struct SegFinalSub {
   AdamScalars s;
   __device__ void operator()(int64_t block, int64_t nblocks) const;
   __device__ void hot(int64_t block) const;
-  __device__ __forceinline__ void emit(int64_t row, int l, int nchunk, const ChunkFrag<NC>& tot) const;
+  __device__ __forceinline__ void emit(int64_t row, int l, int nchunk, const RowFrag<4 * NC>& tot) const;
 };
 
 template <int LPR, int NC, int MODE, bool WIN>
 __device__ __forceinline__ void SegFinalSub<LPR, NC, MODE, WIN>::emit(int64_t row, int l, int nchunk,
-                                                                      const ChunkFrag<NC>& tot) const {
+                                                                      const RowFrag<4 * NC>& tot) const {
   if (MODE == 0) {
     chunk_store<LPR, NC>(out + row * D, l, nchunk, tot);
   } else {
     float* rec = out + row * 3 * D;
-    ChunkFrag<NC> w = chunk_load<LPR, NC, false>(rec, l, nchunk),
+    RowFrag<4 * NC> w = chunk_load<LPR, NC, false>(rec, l, nchunk),
                   m = chunk_load<LPR, NC, false>(rec + D, l, nchunk),
                   v = chunk_load<LPR, NC, false>(rec + 2 * D, l, nchunk);
-    chunk_adam<NC>(w, m, v, tot, s);
+    frag_adam<4 * NC>(w, m, v, tot, s);
     chunk_store<LPR, NC>(rec, l, nchunk, w);
     chunk_store<LPR, NC>(rec + D, l, nchunk, m);
     chunk_store<LPR, NC>(rec + 2 * D, l, nchunk, v);
@@ -1057,7 +1032,7 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
     const int64_t nr = WIN ? L : (L + kAtenGroup - 1) / kAtenGroup;   // rows to add: gradients, or run sums
     const f32x4* src = reinterpret_cast<const f32x4*>(
         WIN ? grad : parts + (int64_t)chunk_off[u] * kGroupsPerChunk * D);
-    ChunkFrag<NC> tot = chunk_zero<NC>(), acc = tot;
+    RowFrag<4 * NC> tot = frag_zero<4 * NC>(), acc = tot;
     int32_t prev = -1;
     for (int64_t r0 = 0; r0 < nr; r0 += per) {
       const int m = (int)(nr - r0 < per ? nr - r0 : per);
@@ -1071,27 +1046,27 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
       __syncthreads();
       if (t < LPR) {
         for (int r = 0; r < m; ++r) {
-          ChunkFrag<NC> x;
+          RowFrag<4 * NC> x;
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             const f32x4 g = t + c * LPR < nchunk ? stage[r * nchunk + t + c * LPR] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) x.v[c][j] = g[j];
+            for (int j = 0; j < 4; ++j) x.v[4 * c + j] = g[j];
           }
           if (!WIN) {
-            chunk_add<NC>(tot, x);
+            frag_add<4 * NC>(tot, x);
           } else if (win[r] != prev) {
-            if (prev >= 0) chunk_add<NC>(tot, acc);
+            if (prev >= 0) frag_add<4 * NC>(tot, acc);
             acc = x;
             prev = win[r];
           } else {
-            chunk_add<NC>(acc, x);
+            frag_add<4 * NC>(acc, x);
           }
         }
       }
     }
     if (t < LPR) {
-      if (WIN) chunk_add<NC>(tot, acc);
+      if (WIN) frag_add<4 * NC>(tot, acc);
       const int64_t row = uniq ? uniq[u] : u;
       if (row >= 0 && row < nrows) emit(row, t, nchunk, tot);
     }
@@ -1113,16 +1088,16 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::operator()(int64_t block, int64
   const int64_t row = uniq ? uniq[u] : u;   // NULL: segment u goes to row u
   const int32_t o0 = seg_occ0[u];
   if (row < 0 || row >= nrows || (WIN ? L > kWinHot : seg_hot(L))) return;   // hot segments: a block's
-  ChunkFrag<NC> acc = chunk_load<LPR, NC, true>(grad + (int64_t)o0 * D, l, nchunk);
+  RowFrag<4 * NC> acc = chunk_load<LPR, NC, true>(grad + (int64_t)o0 * D, l, nchunk);
   float* rec = out + row * 3 * D;
-  ChunkFrag<NC> w, m, v;
+  RowFrag<4 * NC> w, m, v;
   if (MODE == 1) {
     w = chunk_load<LPR, NC, false>(rec, l, nchunk);
     m = chunk_load<LPR, NC, false>(rec + D, l, nchunk);
     v = chunk_load<LPR, NC, false>(rec + 2 * D, l, nchunk);
   }
   const int inl = (int)(WIN ? L : (L < kSegChunk ? L : kSegChunk));
-  ChunkFrag<NC> tot = chunk_zero<NC>();
+  RowFrag<4 * NC> tot = frag_zero<4 * NC>();
   int32_t prev = o0;
   int in_run = 1;   // occurrences of the open run (sort path)
   constexpr int R = kSubRows<NC>;
@@ -1131,7 +1106,7 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::operator()(int64_t block, int64
   for (int e = 0; e < R; ++e) o[e] = sv[s0 + (1 + e < inl ? 1 + e : 0)];
   for (int k0 = 1; k0 < inl; k0 += R) {
     // this batch's rows, then the next batch's indices, so that a batch costs one round trip
-    ChunkFrag<NC> g[R];
+    RowFrag<4 * NC> g[R];
     int32_t on[R];
 #pragma unroll
     for (int e = 0; e < R; ++e) g[e] = chunk_load<LPR, NC, true>(grad + (int64_t)o[e] * D, l, nchunk);
@@ -1142,11 +1117,11 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::operator()(int64_t block, int64
       if (k0 + e >= inl) continue;
       const bool head = WIN ? (o[e] >> kAtenWinShift) != (prev >> kAtenWinShift) : in_run == kAtenGroup;
       if (head) {
-        chunk_add<NC>(tot, acc);
+        frag_add<4 * NC>(tot, acc);
         acc = g[e];
         in_run = 1;
       } else {
-        chunk_add<NC>(acc, g[e]);
+        frag_add<4 * NC>(acc, g[e]);
         ++in_run;
       }
       prev = o[e];
@@ -1154,24 +1129,24 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::operator()(int64_t block, int64
 #pragma unroll
     for (int e = 0; e < R; ++e) o[e] = on[e];
   }
-  chunk_add<NC>(tot, acc);
+  frag_add<4 * NC>(tot, acc);
   if (!WIN && L > kSegChunk) {
     const int np = (int)((L - kSegChunk + kAtenGroup - 1) / kAtenGroup);
     const float* pr = parts + (int64_t)chunk_off[u] * kGroupsPerChunk * D;
     for (int c0 = 0; c0 < np; c0 += kSubRows<NC>) {
-      ChunkFrag<NC> pc[kSubRows<NC>];
+      RowFrag<4 * NC> pc[kSubRows<NC>];
 #pragma unroll
       for (int e = 0; e < kSubRows<NC>; ++e)
         pc[e] = chunk_load<LPR, NC, false>(pr + (int64_t)(c0 + e < np ? c0 + e : c0) * D, l, nchunk);
 #pragma unroll
       for (int e = 0; e < kSubRows<NC>; ++e)
-        if (c0 + e < np) chunk_add<NC>(tot, pc[e]);
+        if (c0 + e < np) frag_add<4 * NC>(tot, pc[e]);
     }
   }
   if (MODE == 0) {
     chunk_store<LPR, NC>(out + row * D, l, nchunk, tot);
   } else {
-    chunk_adam<NC>(w, m, v, tot, s);
+    frag_adam<4 * NC>(w, m, v, tot, s);
     chunk_store<LPR, NC>(rec, l, nchunk, w);
     chunk_store<LPR, NC>(rec + D, l, nchunk, m);
     chunk_store<LPR, NC>(rec + 2 * D, l, nchunk, v);

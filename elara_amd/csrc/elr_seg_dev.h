@@ -3,8 +3,6 @@
 // and its occurrence gradients.
 #pragma once
 
-#include <type_traits>
-
 #include "elr_launch.h"
 #include "elr_rowio.h"
 
@@ -95,63 +93,7 @@ __device__ void SegPartials<NQ>::operator()(int64_t blk, int64_t nblk) const {
   }
 }
 
-// Rows of 16-byte chunks spread over groups of lanes: LPR lanes (a power of two) take one row, lane l of a group its
-// chunks l, l + LPR, ... (NC of them), so a wave works on 64 / LPR rows at once and every load is 16 bytes a lane.
-// For widths that are a multiple of 4; LPR covers the row's D / 4 chunks where that is at most 64.
-template <int NC>
-struct ChunkFrag {
-  float v[NC][4];
-};
-
-// Loads are unconditional: a chunk past the row's end loads chunk 0 instead (its lanes compute what chunk 0's lanes do
-// and store nothing).  A load under a per-lane condition ends in a branch with a wait, which serialises the loads of
-// a batch of rows (the final segment kernel at 107k occurrences of width 48: 29 us that way, 26 without).
-template <int LPR, int NC, bool NT>
-__device__ __forceinline__ ChunkFrag<NC> chunk_load(const float* __restrict__ row, int l, int nchunk) {
-  ChunkFrag<NC> r;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int q = l + c * LPR;
-    const f32x4* p = reinterpret_cast<const f32x4*>(row) + (q < nchunk ? q : 0);
-    const f32x4 t = NT ? __builtin_nontemporal_load(p) : *p;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r.v[c][j] = t[j];
-  }
-  return r;
-}
-
-template <int LPR, int NC, bool NT = true>
-__device__ __forceinline__ void chunk_store(float* __restrict__ row, int l, int nchunk, const ChunkFrag<NC>& x) {
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const f32x4 t = {x.v[c][0], x.v[c][1], x.v[c][2], x.v[c][3]};
-    if (l + c * LPR < nchunk) {
-      f32x4* p = reinterpret_cast<f32x4*>(row) + l + c * LPR;
-      if (NT) __builtin_nontemporal_store(t, p);
-      else *p = t;
-    }
-  }
-}
-
-template <int NC>
-__device__ __forceinline__ void chunk_add(ChunkFrag<NC>& a, const ChunkFrag<NC>& b) {
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a.v[c][j] = a.v[c][j] + b.v[c][j];
-}
-
-template <int NC>
-__device__ __forceinline__ ChunkFrag<NC> chunk_zero() {
-  ChunkFrag<NC> z;
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) z.v[c][j] = 0.0f;
-  return z;
-}
-
-// SegPartials in that layout: a group of lanes sums one run (its ten rows load together), so a wave has 64 / LPR runs
+// SegPartials in the chunk layout (elr_rowio.h): a group of lanes sums one run (its ten rows load together), so a wave has 64 / LPR runs
 // in flight (5.1 us against 7.4 for a wave per chunk at width 48, 107k
 // occurrences).
 template <int LPR, int NC>
@@ -175,14 +117,14 @@ __device__ void SegPartialsSub<LPR, NC>::operator()(int64_t blk, int64_t nblk) c
     int32_t o[kAtenGroup];
 #pragma unroll
     for (int r = 0; r < kAtenGroup; ++r) o[r] = a.sv[r < len ? p0 + r : p0];
-    ChunkFrag<NC> g[kAtenGroup];
+    RowFrag<4 * NC> g[kAtenGroup];
 #pragma unroll
     for (int r = 0; r < kAtenGroup; ++r)
       g[r] = chunk_load<LPR, NC, true>(a.grad + (int64_t)o[r] * a.D, l, nchunk);
-    ChunkFrag<NC> acc = g[0];
+    RowFrag<4 * NC> acc = g[0];
 #pragma unroll
     for (int r = 1; r < kAtenGroup; ++r)
-      if (r < len) chunk_add<NC>(acc, g[r]);
+      if (r < len) frag_add<4 * NC>(acc, g[r]);
     chunk_store<LPR, NC, false>(a.parts + q * a.D, l, nchunk, acc);
   }
 }
@@ -223,31 +165,6 @@ struct DirLstepsHits;   // elr_dir_dev.h
 int segment_sum_plan_final_with(const float* grad, int64_t n, int64_t D, int key_bits, const void* plan,
                                 int64_t plan_bytes, const int64_t* perm, float* out, int64_t out_rows,
                                 const DirLstepsHits& first, int64_t nb1, void* stream);
-
-// Lanes per row of the chunk layout for width D (a multiple of 4, at most 512): D / 4 rounded up to a power of two of
-// at least 4, at most 64; 0 for other widths and unaligned arrays.
-inline int chunk_lanes(int64_t D, const void* a, const void* b) {
-  if (D % 4 || D > 512 || !aligned16(a) || !aligned16(b)) return 0;
-  int l = 4;
-  while (l < D / 4 && l < 64) l *= 2;
-  return l;
-}
-
-// visit(lanes per row, chunks per lane) as integral constants, for chunk_lanes' value lpr.
-template <class Visit>
-inline void chunk_visit(int lpr, int64_t D, Visit&& visit) {
-  using std::integral_constant;
-  switch (lpr) {
-    case 4: visit(integral_constant<int, 4>{}, integral_constant<int, 1>{}); break;
-    case 8: visit(integral_constant<int, 8>{}, integral_constant<int, 1>{}); break;
-    case 16: visit(integral_constant<int, 16>{}, integral_constant<int, 1>{}); break;
-    case 32: visit(integral_constant<int, 32>{}, integral_constant<int, 1>{}); break;
-    default:
-      if (D <= 256) visit(integral_constant<int, 64>{}, integral_constant<int, 1>{});
-      else visit(integral_constant<int, 64>{}, integral_constant<int, 2>{});
-      break;
-  }
-}
 
 template <class Visit>
 inline void seg_partials_visit(const SegPartialsLaunch& L, Visit&& visit) {

@@ -5,14 +5,15 @@
 //        scalars of logical step steps[i,k] and the gradient logs[offs[i]+k].  The Adam arithmetic is
 //        elr::adam_elem, so replay(init, log) is bitwise equal to eager Adam applied at those steps.
 //
-// D in {64, 128, 256, 512}: wave-per-row kernels (elr_rowio.h).  A wave owns U rows; their ids, counts, log offsets
+// D in {128, 256}, and 64 for init: wave-per-row kernels (elr_rowio.h).  A wave owns U rows; their ids, counts, log offsets
 // and steps are scalar loads, all their log-entry loads are issued before the first update, the Adam scalars of each
 // step come through the scalar cache, the initial weights are computed in registers while the loads are in
 // flight, and each record is written once.  The kernels have no loop: a loop back-edge makes the compiler guard the
 // next iteration's loads with vmcnt(0) waits that also drain this iteration's stores, so very large calls are split
 // into several launches on the host instead.
-// Other D, or no reciprocal table: the generic kernels below (2^lg lanes per row with 16-byte chunks, or one float
-// per lane).
+// Replay at other D up to 512 that are a multiple of 4: the chunk layout (elr_rowio.h), several rows per wave.  Init at
+// other D, wider rows or no reciprocal table: the generic kernels below (2^lg lanes per row with 16-byte chunks, or one
+// float per lane).
 #include "elr_rowio.h"
 
 namespace elr {
@@ -278,23 +279,95 @@ static void launch_init_wpr(float* out, const int64_t* rows, int64_t n, uint32_t
   }
 }
 
+// ---- chunk layout (elr_rowio.h): 64 / LPR rows per wave -----------------------------------------------------------
+// A row's metadata, steps and scalars are per group of lanes here (vector loads that hit the cache, where the wave per
+// row reads them as scalars); every row's log entries load together, then the arithmetic of k_replay_wpr: the cores
+// for every step, one range check per row, and a recompute on the general path where a lane fails it.  Against a wave per row
+// with 4 bytes a lane, or the generic kernel's range check and branch per element: 54 against 71 us at 200,000 rows of
+// width 64 (K = 3), 41 against 60 at 300,000 of 32, 78 against 124 at 100,000 of 200, 68 against 80 at 40,000 of 512;
+// 128 and 256 stay a wave per row (91 against 102 us, 82 against 84).
+template <int LPR, int NC, int K>
+__global__ __launch_bounds__(256) void k_replay_sub(float* __restrict__ out, const int64_t* __restrict__ rows,
+                                                    const float* __restrict__ logs, int64_t nlogs,
+                                                    const int64_t* __restrict__ offs,
+                                                    const int32_t* __restrict__ steps,
+                                                    const int32_t* __restrict__ cnt, int64_t n, int64_t D,
+                                                    uint32_t seed, float bound, const float* __restrict__ table,
+                                                    const double* __restrict__ recip, int64_t table_rows) {
+  constexpr int GPW = 64 / LPR;
+  const int lane = threadIdx.x & 63, l = lane & (LPR - 1), nchunk = (int)(D / 4);
+  const int64_t i = wave_id() * GPW + lane / LPR;
+  if (i >= n) return;
+  const int64_t r = rows[i], o = offs[i];
+  const int ci = cnt[i], c = ci < 0 ? 0 : (ci > K ? K : ci);
+  int32_t st[K];
+  // every used step indexes the table and every used log entry exists, or the row is skipped
+  int bad = (o < 0) | (o + c > nlogs);
+#pragma unroll
+  for (int k = 0; k < K; ++k) st[k] = steps[i * K + k];
+#pragma unroll
+  for (int k = 0; k < K; ++k) bad |= (k < c) & ((st[k] < 0) | (st[k] >= table_rows));
+  if (bad) return;
+  RowFrag<4 * NC> g[K];
+  AdamScalars sc[K];
+  if (nlogs > 0 && table_rows > 0) {   // (entries past a row's count load entry 0 and step 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      g[k] = chunk_load<LPR, NC, true>(logs + (k < c ? o + k : 0) * D, l, nchunk);
+      sc[k] = table_scalars(table, recip, k < c ? st[k] : 0);
+    }
+  }
+  RowFrag<4 * NC> w = chunk_init<LPR, NC>(r, D, l, seed, bound), m = frag_zero<4 * NC>(), v = frag_zero<4 * NC>();
+  RangeAcc acc = range_acc_init();
+  bool eps_all = true;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (k < c) {
+      eps_all = eps_all && eps_ok(sc[k].eps);
+      frag_adam_fast<4 * NC>(w, m, v, g[k], sc[k], acc);
+    }
+  if (!wave_all(eps_all && range_acc_ok(acc))) {
+    w = chunk_init<LPR, NC>(r, D, l, seed, bound);
+    m = frag_zero<4 * NC>();
+    v = frag_zero<4 * NC>();
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (k < c) frag_adam<4 * NC>(w, m, v, g[k], sc[k]);
+  }
+  float* dst = out + i * 3 * D;
+  chunk_store<LPR, NC>(dst, l, nchunk, w);
+  chunk_store<LPR, NC>(dst + D, l, nchunk, m);
+  chunk_store<LPR, NC>(dst + 2 * D, l, nchunk, v);
+}
+
 template <int K>
 static int launch_replay(float* out, const int64_t* rows, const float* logs, int64_t nlogs, const int64_t* offs,
                          const int32_t* steps, const int32_t* cnt, int64_t n, int64_t D, uint32_t seed, float bound,
                          const float* table, const double* recip, int64_t table_rows, hipStream_t st, hipEvent_t e0,
                          hipEvent_t e1) {
   const int vpl = wpr_vpl(D);
-  if (K <= 4 && vpl && recip && aligned16(out) && aligned16(logs)) {
+  if ((vpl == 2 || vpl == 4) && recip && aligned16(out) && aligned16(logs)) {
 #define ELR_WPR_REPLAY(V) \
   launch_replay_wpr<V, K>(out, rows, logs, nlogs, offs, steps, cnt, n, seed, bound, table, recip, table_rows, st, \
                           e0, e1)
     switch (vpl) {
-      case 1: ELR_WPR_REPLAY(1); break;
       case 2: ELR_WPR_REPLAY(2); break;
-      case 4: ELR_WPR_REPLAY(4); break;
-      default: ELR_WPR_REPLAY(8); break;
+      default: ELR_WPR_REPLAY(4); break;
     }
 #undef ELR_WPR_REPLAY
+    return launch_status();
+  }
+  if (const int lpr = recip ? chunk_lanes(D, out, logs) : 0) {
+    chunk_visit(lpr, D, [&](auto L_, auto N_) {
+      constexpr int LPR = L_.value, NC = N_.value, GPW = 64 / LPR;
+      constexpr int64_t per = wpr_rows_per_launch(GPW);
+      for (int64_t a = 0; a < n; a += per) {
+        const int64_t m = n - a < per ? n - a : per;
+        launch_timed(k_replay_sub<LPR, NC, K>, grid_for((m + GPW - 1) / GPW, 4, kOneShotBlocks), st,
+                     a == 0 ? e0 : nullptr, a + m >= n ? e1 : nullptr, out + a * 3 * D, rows + a, logs, nlogs, offs + a,
+                     steps + a * K, cnt + a, m, D, seed, bound, table, recip, table_rows);
+      }
+    });
     return launch_status();
   }
   if (D % 4 == 0 && D / 4 <= INT32_MAX && aligned16(out) && aligned16(logs) && aligned16(table)) {
@@ -319,12 +392,13 @@ extern "C" int elr_init_rows(float* out, const int64_t* rows, int64_t n, int64_t
   if (!out || !rows) return ELR_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   const int vpl = elr::wpr_vpl(D);
-  if (vpl && elr::aligned16(out)) {
+  // (D = 512 is not a wave's row here: a lane's two 16-byte stores would lie 32 bytes apart, half a line each, and
+  // writes alone show it: 120,000 rows 316 us against 137 in chunks of 64 lanes)
+  if (vpl && vpl < 8 && elr::aligned16(out)) {
     switch (vpl) {
       case 1: elr::launch_init_wpr<1>(out, rows, n, seed, bound, st); break;
       case 2: elr::launch_init_wpr<2>(out, rows, n, seed, bound, st); break;
-      case 4: elr::launch_init_wpr<4>(out, rows, n, seed, bound, st); break;
-      default: elr::launch_init_wpr<8>(out, rows, n, seed, bound, st); break;
+      default: elr::launch_init_wpr<4>(out, rows, n, seed, bound, st); break;
     }
   } else if (D % 4 == 0 && D / 4 <= INT32_MAX && elr::aligned16(out)) {
     const int64_t nchunk = D / 4;

@@ -325,3 +325,45 @@ def test_gpu_adam_check_raises_on_rows_out_of_range(dev):
     adam_dedup(pool, torch.tensor([1, 1, 2], device=dev), g, *synth.ADAM, 1, check=True)
     torch.cuda.synchronize()
     assert pool[[0, 4, 9, 1, 2], 0].ne(0).all() and not pool[[3, 5, 6, 7, 8]].any()
+
+
+@pytest.mark.parametrize('n', [1, 2, 33, 4_099])
+@pytest.mark.parametrize('D', [4, 12, 16, 24, 48, 96, 320, 516])
+def test_rows_in_chunk_layout(dev, D, n):
+    """Adam, init and replay at widths whose rows move in 16-byte chunks, several rows per wave (every number of lanes per
+    row, two chunks per lane, and one width past it): partly filled waves, slots out of range, rows whose gradients
+    leave the fast arithmetic's range beside rows that stay in it, empty logs; bitwise the oracle's."""
+    step_banner(f'chunk layout D={D} n={n}')
+    rng = np.random.default_rng(D + n)
+    seed, bound = 77, 0.05
+    rows = rng.integers(0, 2**35, n).astype(np.int64)
+    got = init_rows(torch.from_numpy(rows).to(dev), D, seed, bound)
+    assert same(got, O.init_rows(rows, D, seed, bound))
+    # Adam: slots out of range are skipped
+    C = 2 * n + 3
+    state = (rng.standard_normal((C, 3, D)) * 0.05).astype(np.float32)
+    state[:, 2] **= 2
+    g = (rng.standard_normal((n, D)) * 1e-3).astype(np.float32)
+    g[rng.random(n) < 0.2] = 0.0
+    g[rng.random(n) < 0.1] *= np.float32(1e30)
+    state[rng.random(C) < 0.2, 1:] = 0.0
+    slots = rng.permutation(C)[:n].astype(np.int64)
+    gpu = torch.from_numpy(state.copy()).to(dev)
+    bad = slots.copy()
+    bad[::5] = np.where(np.arange(bad[::5].size) % 2 == 0, -1, C)
+    gpu_adam(gpu, torch.from_numpy(bad).to(dev), torch.from_numpy(g).to(dev), *HP, 7)
+    keep = (bad >= 0) & (bad < C)
+    O.cpu_adam(state, slots[keep], g[keep], O.adam_scalars(*HP, 7), 2)
+    assert same(gpu, state)
+    for K in (3, 6):
+        cnt = rng.integers(0, K + 1, n).astype(np.int32)
+        if n == 1:
+            cnt[:] = 0   # an empty log
+        steps = np.cumsum(rng.integers(1, 30, (n, K)), 1).astype(np.int32)
+        offs = (np.cumsum(cnt) - cnt).astype(np.int64)
+        logs = (rng.standard_normal((int(cnt.sum()), D)) * 1e-3).astype(np.float32)
+        logs[rng.random(logs.shape[0]) < 0.2] = 0.0
+        table = ScalarTable(*HP, 30 * K, dev)
+        t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+        rp = replay_rows(t(rows), t(logs), t(offs), t(steps), t(cnt), D, K, seed, bound, table)
+        assert same(rp, O.replay_rows(rows, logs, offs, steps, cnt, D, K, seed, bound, table.t.cpu().numpy()))
