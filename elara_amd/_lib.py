@@ -225,6 +225,32 @@ def lib():
     return _lib
 
 
+NOT_TAKEN = -1000   # _hostcall's answer for arguments the Python path has to look at
+
+
+class _NoHost:
+    """Stands in for _hostcall where it is not built for this interpreter's torch: the Python path takes every call."""
+    adam = init = replay = staticmethod(lambda *a: NOT_TAKEN)
+
+
+_host = None
+
+
+def host():
+    """The native argument checks of the row ops (csrc/hostcall.cpp), bound to the loaded library."""
+    global _host
+    if _host is None:
+        L = lib()
+        try:
+            from . import _hostcall as h
+            h.bind(*(ctypes.cast(f, c_vp).value for f in (L.elr_adam_scalars, L.elr_adam_rows, L.elr_init_rows,
+                                                          L.elr_replay_rows)))
+        except ImportError:
+            h = _NoHost
+        _host = h
+    return _host
+
+
 def check(rc, what):
     """Raise RuntimeError for a nonzero C-ABI return code (the reference raises through TORCH_CHECK)."""
     if rc != 0:

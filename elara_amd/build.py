@@ -1,9 +1,9 @@
 """Build recipe of libelara_amd.so (hipcc, gfx950 only).
 
 Every .hip file under csrc/ is compiled on its own (in parallel) and linked into one shared library next to this
-file.  Float flags: no FMA contraction, correctly rounded fp32 division and square root, denormals kept -- the
-conditions under which the kernels are bitwise equal to the reference's CPU Adam.  Packed-fp32 instructions are
-disabled for device code.
+file; csrc/hostcall.cpp, the Python side's native argument checks, becomes the extension module _hostcall.  Float
+flags: no FMA contraction, correctly rounded fp32 division and square root, denormals kept -- the conditions under
+which the kernels are bitwise equal to the reference's CPU Adam.  Packed-fp32 instructions are disabled for device code.
 """
 import os
 import subprocess
@@ -14,6 +14,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / 'csrc'
 LIB = HERE / 'libelara_amd.so'
+HOST_SRC, HOST_LIB = CSRC / 'hostcall.cpp', HERE / '_hostcall.so'
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 ARCH = 'gfx950'
 
@@ -47,14 +48,32 @@ def _compile(src, obj):
     return obj
 
 
+def _build_host():
+    """The extension module _hostcall (host code only) against this interpreter's torch."""
+    import sysconfig
+    import torch
+    inc, lib = Path(torch.__file__).parent / 'include', Path(torch.__file__).parent / 'lib'
+    tmp = HOST_LIB.with_suffix('.so.tmp')
+    cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-D__HIP_PLATFORM_AMD__=1',
+           '-DUSE_ROCM', f'-I{inc}', f'-I{inc}/torch/csrc/api/include', '-I/opt/rocm/include',
+           f'-I{sysconfig.get_paths()["include"]}', str(HOST_SRC), '-o', str(tmp), f'-L{lib}', '-ltorch_python',
+           '-ltorch_cpu', '-lc10', '-lc10_hip']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f'{HOST_SRC.name} failed:\n{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
+    os.replace(tmp, HOST_LIB)
+
+
 def build(verbose=False):
-    """Compile every kernel source and link libelara_amd.so (always rebuilds)."""
+    """Compile every kernel source and link libelara_amd.so, and the host module (always rebuilds)."""
     objdir = HERE / '_build'
     objdir.mkdir(exist_ok=True)
     srcs = sources()
     objs = [objdir / (s.stem + '.o') for s in srcs]
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(_build_host)
         list(ex.map(_compile, srcs, objs))
+        host.result()
     tmp = LIB.with_suffix('.so.tmp')
     cmd = [HIPCC, '-shared', f'--offload-arch={ARCH}', '-o', str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)

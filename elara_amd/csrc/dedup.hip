@@ -594,7 +594,7 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(Keys keys, const Key* _
 // come from the general path's two launches (k_seg_count, k_seg_apply with FieldKeys), so the plan is the general
 // path's, bit for bit, in four launches.  A thread holds as many keys as the column needs (1 to 16).  (The
 // segments by one block per field, as the sort's, took 28 us of a 26-column batch of 426k; the two launches over
-// the whole GPU FIELDSEG.)  An id outside its field's rows takes the key R_c (the field's row count), sorts after the
+// the whole GPU 18, and the whole plan 104 -> 76.)  An id outside its field's rows takes the key R_c (the field's row count), sorts after the
 // field's ids and comes out as -1 in uniq: a row out of range for the caller.
 constexpr int kFieldThreads = 1024;
 constexpr int kFieldItems = 16;
@@ -742,7 +742,10 @@ __global__ __launch_bounds__(kFieldThreads) void k_field_sort(const uint32_t* __
 
 // The whole dedup plan of at most kFieldThreads * ITEMS ids by one block: the sort in LDS, the segment heads from
 // ballots, the inverse, the hot segments and the partial-chunk plan -- what the radix passes, k_seg_count and
-// k_seg_apply leave, in one launch.  SMALLPLAN
+// k_seg_apply leave, in one launch.  Against the general path's ten launches of 2 to 5 us each, every one waiting for
+// the one before, one block's passes over LDS are the shorter chain: 12.8 us at 2,600 ids, and the whole update of a
+// batch of 2,600 36.4 -> 17.8 us.  The line: whole updates of 7,800 ids 40.0 -> 35.1 and of 8,000 ids 58 -> 43 us by
+// this kernel, its time growing with the ids while the general path's barely does.
 constexpr int kSmallItems = 8;
 constexpr int64_t kSmallPlan = kFieldThreads * kSmallItems;
 template <typename Key, int ITEMS>

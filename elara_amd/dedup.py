@@ -17,6 +17,8 @@ zeroed row; above 3072, an id's occurrences in ascending index are cut into runs
 and the run sums added from zero.  Equal bits to torch.ops.aten.embedding_dense_backward on the same inputs.  All
 of it runs as HIP kernels (elara_amd/csrc/dedup.hip) on torch's current stream.
 """
+import functools
+
 import torch
 
 from . import _lib
@@ -50,8 +52,9 @@ def _bits(bound):
 def _key_bits(flat, bound):
     if bound is not None:
         return _bits(int(bound))
-    lo, hi = torch.aminmax(flat)
-    lo, hi = int(lo), int(hi)
+    mm = torch.empty(2, dtype=I64, device=flat.device)
+    torch.aminmax(flat, out=(mm[0], mm[1]))
+    lo, hi = mm.tolist()   # one read for both
     if lo < 0:
         raise RuntimeError('unique: ids must be non-negative')
     return _bits(hi + 1)
@@ -104,6 +107,7 @@ def unique_plan(ids, D, bound=None, fields=None):
     return u, plan
 
 
+@functools.lru_cache(maxsize=256)
 def plan_bytes(n, D):
     """Bytes of the plan buffer of a batch of n ids for gradients of width D (elr_dedup_plan_bytes)."""
     nbytes = int(_lib.lib().elr_dedup_plan_bytes(int(n), int(D)))
@@ -112,7 +116,7 @@ def plan_bytes(n, D):
     return nbytes
 
 
-def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None):
+def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None, stream=None):
     """unique_plan without reading the unique count: returns (u_full, plan, nu) with u_full [n] whose first nu
     entries are the unique ids, nu the count on the device (None when n == 0).  Set plan.U once nu is known.
     nu_out (int64 [1] on the device, optional): where the count goes, else a new tensor.
@@ -122,8 +126,12 @@ def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None):
     fields (optional, field_bounds(...)): the batch is laid out by field -- (sample, field) order, field c's ids in
     [fields[c], fields[c + 1]) -- and is sorted per field (elr_dedup_plan_fields): the same plan, in three launches.
     An id outside its field's rows comes out as -1 in u.  Batches whose size is not a multiple of the field count
-    take the general sort."""
+    take the general sort.
+    stream (optional, with bound and out): the stream the plan is queued on instead of the current one; ids must then
+    be contiguous int64 (nothing is converted on the current stream)."""
     flat = _ids(ids)
+    if stream is not None and (bound is None or out is None or flat.data_ptr() != ids.data_ptr()):
+        raise RuntimeError('unique_plan_async: stream needs bound, out and contiguous int64 ids')
     n = flat.numel()
     dev = flat.device
     plan = DedupPlan()
@@ -150,15 +158,16 @@ def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None):
         raise RuntimeError(f'nu_out must be an int64 tensor of one element on {dev}')
     nu = nu_out if nu_out is not None else torch.empty(1, dtype=I64, device=dev)
     nf = 0 if fields is None else fields.size - 1
+    st = _lib.stream_of(flat) if stream is None else stream.cuda_stream
     with _lib.on_device(dev):
         if nf > 0 and n % nf == 0:
             rc = _lib.lib().elr_dedup_plan_fields(_lib.ptr(flat), n // nf, nf, fields.ctypes.data, plan.key_bits,
                                                   _lib.ptr(u), None, _lib.ptr(nu), _lib.ptr(plan.buf), nbytes, int(D),
-                                                  _lib.stream_of(flat))
+                                                  st)
             _lib.check(rc, 'elr_dedup_plan_fields')
             return u, plan, nu
         rc = _lib.lib().elr_dedup_plan(_lib.ptr(flat), n, plan.key_bits, _lib.ptr(u), None, _lib.ptr(nu),
-                                       _lib.ptr(plan.buf), nbytes, int(D), _lib.stream_of(flat))
+                                       _lib.ptr(plan.buf), nbytes, int(D), st)
     _lib.check(rc, 'elr_dedup_plan')
     return u, plan, nu
 

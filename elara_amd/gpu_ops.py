@@ -19,6 +19,11 @@ def _seed32(seed):
 
 def init_rows(rows, D, seed, bound, out=None):
     """rows: cuda int64 [n] -> out [n,3,D] (w0, 0, 0).  Allocates `out` when None."""
+    if out is None:
+        r = (_lib._host or _lib.host()).init(rows, D, seed, bound)
+        if r != _lib.NOT_TAKEN:
+            _lib.check(r[0], 'elr_init_rows')
+            return r[1]
     n = rows.numel()
     if out is None:
         out = torch.empty(n, 3, D, device=rows.device)
@@ -58,6 +63,11 @@ def replay_rows(rows, logs, offs, steps, cnt, D, K, seed, bound, table, out=None
     table: ScalarTable (or its [S,8] tensor) -> out [n,3,D].  Allocates `out` when None.  events: optional
     (start, stop) hipEvent_t handles (integers) that the launch itself records at the kernel's start and end
     (elr_replay_rows_timed); not recorded when n == 0."""
+    if out is None and events is None and type(table) is ScalarTable:
+        r = (_lib._host or _lib.host()).replay(rows, logs, offs, steps, cnt, D, K, seed, bound, table.t, table.r)
+        if r != _lib.NOT_TAKEN:
+            _lib.check(r[0], 'elr_replay_rows')
+            return r[1]
     n = rows.numel()
     if out is None:
         out = torch.empty(n, 3, D, device=rows.device)

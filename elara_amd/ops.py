@@ -93,6 +93,10 @@ def gpu_adam(pool, slots, grad, lr, b1, b2, eps, step, events=None, check=False)
     itself records at the kernel's start and end (elr_adam_rows_timed); not recorded when n == 0.  A slot outside
     [0, C) is skipped by the kernel (the reference leaves it undefined); check=True raises IndexError for it first,
     at the cost of a host synchronisation."""
+    if events is None and not check:
+        rc = (_lib._host or _lib.host()).adam(pool, slots, grad, lr, b1, b2, eps, step)
+        if rc != _lib.NOT_TAKEN:
+            return _lib.check(rc, 'elr_adam_rows')
     n = slots.numel()
     if n == 0:
         return

@@ -75,8 +75,8 @@ class HipBackend:
     def unique(self, ids, bound=None):
         return unique_plan(ids, self.D, bound)
 
-    def unique_async(self, ids, bound=None, nu_out=None, out=None, fields=None):
-        return unique_plan_async(ids, self.D, bound, nu_out, out, fields)
+    def unique_async(self, ids, bound=None, nu_out=None, out=None, fields=None, stream=None):
+        return unique_plan_async(ids, self.D, bound, nu_out, out, fields, stream)
 
     def plan_bytes(self, n):
         return plan_bytes(n, self.D)
@@ -228,8 +228,13 @@ class HipBackend:
             a.mark_value, a.mark_bit = int(mval), int(mbit)
             a.mark_event = mev.cuda_event if mev is not None else None
         L = _lib.lib()
-        nb = int(L.elr_step_dev_bytes(ctypes.byref(a)))
-        _lib.check(min(nb, 0), 'elr_step_dev_bytes')
+        nb = st['bytes'].get(a.plan.n)   # the rest of what the size depends on is fixed for an ElaraStep
+        if nb is None:
+            nb = int(L.elr_step_dev_bytes(ctypes.byref(a)))
+            _lib.check(min(nb, 0), 'elr_step_dev_bytes')
+            if len(st['bytes']) > 256:
+                st['bytes'].clear()
+            st['bytes'][a.plan.n] = nb
         if st['ws'] is None or st['ws'].numel() < nb:
             st['ws'] = torch.empty(nb, dtype=torch.uint8, device=dev)
         ws = st['ws']
@@ -275,7 +280,7 @@ class HipBackend:
         up.logs, up.log_rows, up.glog, up.glog_slots = logs, es.logs.shape[0], glog, es.glog.shape[0]
         up.lr, up.b1, up.b2, up.eps = self.hp
         e.dir_order = 1 if es.dir_impl == 'triton' else 0
-        return {'es': es, 'args': a, 'ws': None, 'seq': 0}
+        return {'es': es, 'args': a, 'ws': None, 'seq': 0, 'bytes': {}}
 
     def step_update(self, es, p, G, part=0):
         """ElaraStep.update in one native call (elr_step_update): the same launches in the same order, issued from
@@ -1175,6 +1180,21 @@ def run(step, batches, grads, steps=None, on_step=None, freeze_gc=True):
         gc.unfreeze()
 
 
+class _CurrentStream:
+    """torch's current stream on a device, the Stream object kept while the raw handle stays the same (asking torch
+    for the object costs several microseconds, and a step asks five times)."""
+    __slots__ = ('dev', 'raw', 'obj')
+
+    def __init__(self, dev):
+        self.dev, self.raw, self.obj = dev, None, None
+
+    def __call__(self):
+        raw = _lib.raw_stream(self.dev)
+        if self.obj is None or raw != self.raw:
+            self.raw, self.obj = raw, torch.cuda.current_stream(self.dev)
+        return self.obj
+
+
 class PlanPool:
     """Reusable dedup-plan buffers for run(): one entry (plan buffer, unique-id array, unique count, and the events
     that order its reuse) per batch between its dedup and its step.  Without it each batch's plan would be new
@@ -1189,6 +1209,7 @@ class PlanPool:
 
     def __init__(self, dev, spare=2):
         self.dev, self.spare = dev, spare
+        self.current = _CurrentStream(dev)
         self.free = []   # entries given back, oldest first
         self.made = 0
 
@@ -1199,13 +1220,13 @@ class PlanPool:
                 if e['rel_set']:
                     side.wait_event(e['rel'])
                 else:   # given back without an event (by a run on one stream): wait for all the main stream's work
-                    side.wait_stream(torch.cuda.current_stream(self.dev))
+                    side.wait_stream(self.current())
             if e['buf'].numel() >= nbytes and e['u'].numel() >= n:
                 return e
             # too small for this batch: new buffers; the old ones go back to the allocator only after the main
             # stream's work on them (they were made on the sort's stream)
             if side is not None:
-                main = torch.cuda.current_stream(self.dev)
+                main = self.current()
                 e['buf'].record_stream(main)
                 e['u'].record_stream(main)
                 e['nu'].record_stream(main)
@@ -1221,7 +1242,7 @@ class PlanPool:
 
     def give(self, e, side):
         if side is not None:
-            e['rel'].record(torch.cuda.current_stream(self.dev))
+            e['rel'].record(self.current())
             e['rel_set'] = True
         self.free.append(e)
 
@@ -1231,6 +1252,7 @@ def _run(step, batches, grads, steps, on_step):
     U, PLANS, AHEAD, ENTRY = {}, {}, {}, {}
     dev = step.d
     side = step.dedup_stream()
+    current = _CurrentStream(dev)
     pool = None
     if dev.type == 'cuda' and getattr(step.be, 'plan_bytes', None) is not None:
         if step._plan_pool is None:
@@ -1260,7 +1282,14 @@ def _run(step, batches, grads, steps, on_step):
         if side is None:
             AHEAD[j] = (*step.be.unique_async(ids, step.R, **kw), None)
             return
-        main = torch.cuda.current_stream(dev)
+        if e is not None and ids is src and ids.dtype == I64 and ids.is_contiguous():
+            # nothing to convert or allocate: the plan's launches go to the side stream by its handle
+            u, dplan, nu = step.be.unique_async(ids, step.R, stream=side, **kw)
+            ev = e['sorted']
+            ev.record(side)
+            AHEAD[j] = (u, dplan, nu, ev)
+            return
+        main = current()
         copied = src.device != ids.device or src.data_ptr() != ids.data_ptr()
         if copied:
             side.wait_stream(main)   # the copy that made ids
@@ -1282,7 +1311,7 @@ def _run(step, batches, grads, steps, on_step):
         step's native call instead, which waits for the sort there."""
         u, dplan, nu, ev = AHEAD.pop(j)
         if ev is not None and not in_next_step:
-            torch.cuda.current_stream(dev).wait_event(ev)
+            current().wait_event(ev)
         PLANS[j] = dplan
         if step.sync_free:   # the device-driven step takes the rows with their count on the device, never read here
             if nu is None:   # an empty batch

@@ -367,3 +367,106 @@ def test_rows_in_chunk_layout(dev, D, n):
         t = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
         rp = replay_rows(t(rows), t(logs), t(offs), t(steps), t(cnt), D, K, seed, bound, table)
         assert same(rp, O.replay_rows(rows, logs, offs, steps, cnt, D, K, seed, bound, table.t.cpu().numpy()))
+
+
+def _forms(dev):
+    """Calls of the row ops in every form their native argument checks look at, as (name, function): valid ones, ones
+    the Python path converts, and ones it refuses."""
+    D, n, K = 24, 50, 3
+    g0 = torch.Generator().manual_seed(5)
+    pool = (torch.randn(80, 3, D, generator=g0) * 0.05).to(dev)
+    pool[:, 2] = pool[:, 2] ** 2
+    slots, grad = torch.randperm(80, generator=g0)[:n].to(dev), (torch.randn(n, D, generator=g0) * 1e-3).to(dev)
+    rows = torch.arange(n, device=dev)
+    cnt = (torch.arange(n, device=dev) % (K + 1)).int()
+    offs, logs = (cnt.cumsum(0) - cnt).long(), (torch.randn(int(cnt.sum()), D, generator=g0) * 1e-3).to(dev)
+    steps = (torch.arange(1, K + 1, device=dev).int()[None, :] * 3).repeat(n, 1)
+    table = ScalarTable(*HP, 20, dev)
+
+    def adam(p=pool, s=slots, g=grad, hp=HP, step=4, **kw):
+        p = p.clone() if torch.is_tensor(p) and not kw.pop('in_place', False) else p
+        r = gpu_adam(p, s, g, *hp, step, **kw)
+        return r, p
+
+    def replay(r=rows, lg=logs, o=offs, st=steps, c=cnt, d=D, k=K, t=table, seed=7, bound=0.05, **kw):
+        return replay_rows(r, lg, o, st, c, d, k, seed, bound, t, **kw)
+    wide = torch.randn(n, 2 * D, device=dev)
+    return [
+        ('adam', adam), ('adam int32', lambda: adam(s=slots.int())), ('adam int16', lambda: adam(s=slots.short())),
+        ('adam flat grad', lambda: adam(g=grad.reshape(-1))), ('adam strided grad', lambda: adam(g=wide[:, :D])),
+        ('adam transposed grad', lambda: adam(g=grad.t().contiguous().t())), ('adam half grad', lambda: adam(g=grad.half())),
+        ('adam short grad', lambda: adam(g=grad[1:])), ('adam cpu grad', lambda: adam(g=grad.cpu())),
+        ('adam cpu slots', lambda: adam(s=slots.cpu())), ('adam 2d pool', lambda: adam(p=pool.reshape(80, -1))),
+        ('adam strided slots', lambda: adam(s=torch.stack([slots, slots], 1)[:, 0])),
+        ('adam strided pool', lambda: adam(p=torch.randn(80, 6, D, device=dev)[:, ::2], in_place=True)),
+        ('adam double pool', lambda: adam(p=pool.double())), ('adam empty', lambda: adam(s=slots[:0], g=grad[:0])),
+        ('adam empty, bad pool', lambda: adam(p=pool.double(), s=slots[:0], g=grad[:0])),
+        ('adam out of range', lambda: adam(s=slots + 60)), ('adam checked', lambda: adam(s=slots + 60, check=True)),
+        ('adam numpy scalars', lambda: adam(hp=tuple(np.float64(x) for x in HP), step=np.int64(4))),
+        ('adam tensor lr', lambda: adam(hp=(torch.tensor(1e-3, dtype=torch.float64), *HP[1:]))),
+        ('adam float step', lambda: adam(step=4.0)), ('adam no step', lambda: adam(step=None)),
+        ('adam huge step', lambda: adam(step=1 << 70)), ('adam negated grad', lambda: adam(g=torch._neg_view(grad))),
+        ('adam grad list', lambda: adam(g=grad.tolist())),
+        ('adam misaligned', lambda: adam(g=torch.cat([grad.reshape(-1), grad[0]])[1:1 + n * D])),
+        ('init', lambda: init_rows(rows, D, 7, 0.05)), ('init int32 rows', lambda: init_rows(rows.int(), D, 7, 0.05)),
+        ('init strided rows', lambda: init_rows(torch.arange(2 * n, device=dev)[::2], D, 7, 0.05)),
+        ('init cpu rows', lambda: init_rows(rows.cpu(), D, 7, 0.05)), ('init empty', lambda: init_rows(rows[:0], D, 7, 0.05)),
+        ('init big seed', lambda: init_rows(rows, D, -3, 0.05)),
+        ('init huge seed', lambda: init_rows(rows, D, 1 << 70, 0.05)),
+        ('init empty, no seed', lambda: init_rows(rows[:0], D, None, 0.05)), ('init no width', lambda: init_rows(rows, 0, 7, 0.05)),
+        ('init out', lambda: init_rows(rows, D, 7, 0.05, out=torch.empty(n, 3, D, device=dev))),
+        ('init 2d rows', lambda: init_rows(rows.reshape(5, -1), D, 7, 0.05)),
+        ('replay', replay), ('replay double logs', lambda: replay(lg=logs.double())),
+        ('replay long steps', lambda: replay(st=steps.long())), ('replay strided cnt', lambda: replay(
+            c=torch.stack([cnt, cnt], 1)[:, 1])), ('replay K mismatch', lambda: replay(k=2)),
+        ('replay K 9', lambda: replay(k=9, st=steps.repeat(1, 3))), ('replay ragged logs', lambda: replay(
+            lg=logs.reshape(-1)[:-1])), ('replay bare table', lambda: replay(t=table.t)),
+        ('replay short offs', lambda: replay(o=offs[1:])),
+        ('replay no entries', lambda: replay(c=torch.zeros_like(cnt), o=torch.zeros_like(offs), lg=logs[:0])),
+        ('replay empty', lambda: replay(r=rows[:0], o=offs[:0], st=steps[:0], c=cnt[:0])),
+    ]
+
+
+def test_native_argument_checks_take_and_refuse_the_same_calls(dev, monkeypatch):
+    """Every form of call through the native argument checks and through the Python path alone: the same results bit by bit,
+    the same exceptions. """
+    from elara_amd import _lib
+    step_banner('native argument checks')
+    assert _lib.host() is not _lib._NoHost
+
+    def outcome(f):
+        try:
+            r = f()
+        except Exception as e:
+            return type(e), str(e)
+        torch.cuda.synchronize()
+        return r
+    native, taken = _lib.host(), set()
+
+    class Spy:
+        pass
+    for name in ('adam', 'init', 'replay'):
+        def call(*a, name=name):
+            r = getattr(native, name)(*a)
+            if r != _lib.NOT_TAKEN:
+                taken.add(current)
+            return r
+        setattr(Spy, name, staticmethod(call))
+    for current, f in _forms(dev):
+        monkeypatch.setattr(_lib, '_host', Spy)
+        a = outcome(f)
+        monkeypatch.setattr(_lib, '_host', _lib._NoHost)
+        b = outcome(f)
+        flat = lambda r: list(r) if isinstance(r, tuple) else [r]  # noqa: E731
+        for x, y in zip(flat(a), flat(b), strict=True):
+            if torch.is_tensor(x) and torch.is_tensor(y):
+                assert x.shape == y.shape and x.dtype == y.dtype and x.device == y.device, current
+                if x.dtype == torch.float32:
+                    assert same(x, y), current
+            else:
+                assert x == y, (current, x, y)
+    assert {'adam', 'adam int32', 'adam flat grad', 'adam out of range', 'adam misaligned', 'init', 'init big seed',
+            'replay', 'replay no entries'} <= taken
+    assert not taken & {'adam strided grad', 'adam half grad', 'adam cpu grad', 'adam double pool', 'adam empty',
+                        'adam float step', 'adam negated grad', 'init int32 rows', 'init cpu rows', 'replay bare table',
+                        'replay double logs', 'replay K mismatch'}
