@@ -594,8 +594,9 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_apply(Keys keys, const Key* _
 // come from the general path's two launches (k_seg_count, k_seg_apply with FieldKeys), so the plan is the general
 // path's, bit for bit, in four launches.  A thread holds as many keys as the column needs (1 to 16).  (The
 // segments by one block per field, as the sort's, took 28 us of a 26-column batch of 426k; the two launches over
-// the whole GPU 18, and the whole plan 104 -> 76.)  An id outside its field's rows takes the key R_c (the field's row count), sorts after the
-// field's ids and comes out as -1 in uniq: a row out of range for the caller.
+// the whole GPU 18, and the whole plan, beside a step's kernels, 104 -> 76.)  An id outside its field's rows takes
+// the key R_c (the field's row count), sorts after the field's ids and comes out as -1 in uniq: a row out of range
+// for the caller.
 constexpr int kFieldThreads = 1024;
 constexpr int kFieldItems = 16;
 constexpr int64_t kFieldRows = (int64_t)kFieldThreads * kFieldItems;   // samples per batch: the row index is 16-bit

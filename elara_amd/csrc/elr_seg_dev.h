@@ -93,9 +93,8 @@ __device__ void SegPartials<NQ>::operator()(int64_t blk, int64_t nblk) const {
   }
 }
 
-// SegPartials in the chunk layout (elr_rowio.h): a group of lanes sums one run (its ten rows load together), so a wave has 64 / LPR runs
-// in flight (5.1 us against 7.4 for a wave per chunk at width 48, 107k
-// occurrences).
+// SegPartials in the chunk layout (elr_rowio.h): a group of lanes sums one run (its ten rows load together), so a
+// wave has 64 / LPR runs in flight (5.1 us against 7.4 for a wave per chunk at width 48, 107k occurrences).
 template <int LPR, int NC>
 struct SegPartialsSub {
   SegPartials<1> a;

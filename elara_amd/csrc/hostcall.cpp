@@ -33,8 +33,8 @@ constexpr int kNotTaken = -1000;
 
 PyObject* not_taken() { return PyLong_FromLong(kNotTaken); }
 
-// A plain dense GPU tensor: no subclass, no functorch or functional wrapper, no lazy negation or conjugation, strided and
-// contiguous.
+// A plain dense GPU tensor: no subclass, no functorch or functional wrapper, no lazy negation or conjugation, strided
+// and contiguous.
 const at::Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);

@@ -5,8 +5,8 @@
 //        scalars of logical step steps[i,k] and the gradient logs[offs[i]+k].  The Adam arithmetic is
 //        elr::adam_elem, so replay(init, log) is bitwise equal to eager Adam applied at those steps.
 //
-// D in {128, 256}, and 64 for init: wave-per-row kernels (elr_rowio.h).  A wave owns U rows; their ids, counts, log offsets
-// and steps are scalar loads, all their log-entry loads are issued before the first update, the Adam scalars of each
+// D in {128, 256}, and 64 for init: wave-per-row kernels (elr_rowio.h).  A wave owns U rows; their ids, counts, log
+// offsets and steps are scalar loads, all their log-entry loads are issued before the first update, the Adam scalars of each
 // step come through the scalar cache, the initial weights are computed in registers while the loads are in
 // flight, and each record is written once.  The kernels have no loop: a loop back-edge makes the compiler guard the
 // next iteration's loads with vmcnt(0) waits that also drain this iteration's stores, so very large calls are split
@@ -282,8 +282,8 @@ static void launch_init_wpr(float* out, const int64_t* rows, int64_t n, uint32_t
 // ---- chunk layout (elr_rowio.h): 64 / LPR rows per wave -----------------------------------------------------------
 // A row's metadata, steps and scalars are per group of lanes here (vector loads that hit the cache, where the wave per
 // row reads them as scalars); every row's log entries load together, then the arithmetic of k_replay_wpr: the cores
-// for every step, one range check per row, and a recompute on the general path where a lane fails it.  Against a wave per row
-// with 4 bytes a lane, or the generic kernel's range check and branch per element: 54 against 71 us at 200,000 rows of
+// for every step, one range check per row, and a recompute on the general path where a lane fails it.  Against a wave
+// per row with 4 bytes a lane, or the generic kernel's range check and branch per element: 54 against 71 us at 200,000 rows of
 // width 64 (K = 3), 41 against 60 at 300,000 of 32, 78 against 124 at 100,000 of 200, 68 against 80 at 40,000 of 512;
 // 128 and 256 stay a wave per row (91 against 102 us, 82 against 84).
 template <int LPR, int NC, int K>
