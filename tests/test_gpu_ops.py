@@ -470,3 +470,26 @@ def test_native_argument_checks_take_and_refuse_the_same_calls(dev, monkeypatch)
     assert not taken & {'adam strided grad', 'adam half grad', 'adam cpu grad', 'adam double pool', 'adam empty',
                         'adam float step', 'adam negated grad', 'init int32 rows', 'init cpu rows', 'replay bare table',
                         'replay double logs', 'replay K mismatch'}
+
+
+@pytest.mark.parametrize('D,K', [(24, 3), (64, 3), (96, 8), (128, 3), (128, 6), (200, 5), (512, 2), (7, 3)])
+def test_replay_rows_without_entries_ignore_their_offset(dev, D, K):
+    """A row with a count of 0 uses no log entry, whatever its offset (a wave per row up to K = 4 wants it in [0, L]): it
+    gets its initial state.  A row with entries outside the logs is skipped."""
+    step_banner(f'replay offsets D={D} K={K}')
+    n, L = 40, 30
+    rows = torch.arange(n, device=dev) * 977
+    cnt = torch.tensor([0, 0, 0, 0, 0, 1, 1, K, K, 1] * (n // 10), dtype=torch.int32, device=dev)
+    big = (1 << 63) - 1
+    free = [0, L, 1, L - 1, L] if D == 128 and K <= 4 else [-1, L + 1, L, big, -big]
+    offs = torch.tensor((free + [-1, L, L - K + 1, big, L - 1]) * (n // 10), device=dev)
+    logs = torch.randn(L, D, generator=torch.Generator().manual_seed(3)).to(dev) * 1e-3
+    steps = torch.arange(1, K + 1, device=dev).int().repeat(n, 1)
+    out = torch.full((n, 3, D), 7.0, device=dev)
+    table = ScalarTable(*HP, 20, dev)
+    replay_rows(rows, logs, offs, steps, cnt, D, K, 5, 0.05, table, out=out)
+    first = init_rows(rows, D, 5, 0.05)
+    last = replay_rows(rows, logs[L - 1:], torch.zeros_like(offs), steps, torch.ones_like(cnt), D, K, 5, 0.05, table)
+    for i in range(n):
+        want = first[i] if i % 10 < 5 else last[i] if i % 10 == 9 else torch.full_like(first[i], 7.0)
+        assert same(out[i], want), i
