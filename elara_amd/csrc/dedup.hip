@@ -83,12 +83,22 @@ inline void sort_plan(int key_bits, int max_bits, int& passes, int& rb) {
   rb = 8;
 }
 
+// The key of a caller's id.  An id outside [0, lim) takes the key lim, which the sort's digits cover and no valid id
+// has (key_lim): digits that cover fewer bits than the whole id would otherwise sort it between the occurrences of a
+// valid id, whose segment it would split in two, and a 32-bit key would cut it to a valid id.  lim == 0: every id is
+// its own key (elr_unique, elr_dedup_plan: the caller's ids lie in [0, 2^key_bits)).
+template <typename Key>
+__device__ __forceinline__ Key key_of(int64_t id, uint64_t lim) {
+  return lim && (uint64_t)id >= lim ? (Key)lim : (Key)id;
+}
+
 // Per-tile histogram of RB-bit digits: digit-major (hist[d * ntile + tile]) for k_radix_hist_scan, tile-major
 // (hist[tile * BINS + d]) when the scatter adds the counts up itself (fold).
 template <typename Src, typename Key, int RB, int NT>
-__global__ __launch_bounds__(NT) void k_radix_hist(const Src* __restrict__ src, int64_t n, int shift,
+__global__ __launch_bounds__(NT) void k_radix_hist(const Src* __restrict__ src, int64_t n, uint64_t lim, int shift,
                                                    int32_t* __restrict__ hist, int64_t ntile, int fold) {
   constexpr int BINS = 1 << RB, ITEMS = kSortTile / NT;
+  constexpr bool FIRST = std::is_same_v<Src, int64_t>;   // the caller's ids
   __shared__ int h[BINS];
   const int t = threadIdx.x;
   const int64_t base = (int64_t)blockIdx.x * kSortTile;
@@ -96,7 +106,8 @@ __global__ __launch_bounds__(NT) void k_radix_hist(const Src* __restrict__ src, 
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     const int64_t pos = base + r * NT + t;
-    kk[r] = pos < n ? (Key)src[pos] : (Key)0;
+    const Src x = pos < n ? src[pos] : (Src)0;
+    kk[r] = FIRST ? key_of<Key>((int64_t)x, lim) : (Key)x;
   }
   for (int b = t; b < BINS; b += NT) h[b] = 0;
   __syncthreads();
@@ -182,7 +193,7 @@ __device__ __forceinline__ void bins_excl_scan(const int (&x)[BPT], Put&& put) {
 template <typename Src, typename Key, bool FIRST, int RB, int NT>
 __global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ src_keys,
                                                                 const int32_t* __restrict__ src_vals, int64_t n,
-                                                                int shift, const int32_t* __restrict__ offs,
+                                                                uint64_t lim, int shift, const int32_t* __restrict__ offs,
                                                                 const int32_t* __restrict__ dtot, int ntile, int fold,
                                                                 Key* __restrict__ dst_keys,
                                                                 int32_t* __restrict__ dst_vals) {
@@ -204,7 +215,8 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ sr
   for (int r = 0; r < ITEMS; ++r) {
     const int64_t pos = base + (int64_t)r * 64 + lane;
     const bool valid = pos < n;
-    kk[r] = valid ? (Key)src_keys[pos] : (Key)0;
+    const Src x = valid ? src_keys[pos] : (Src)0;
+    kk[r] = FIRST ? key_of<Key>((int64_t)x, lim) : (Key)x;
     vv[r] = valid ? (FIRST ? (int32_t)pos : src_vals[pos]) : 0;
   }
   const bool own = t * BPT < BINS;   // this thread's digits
@@ -317,8 +329,11 @@ __device__ __forceinline__ int block_wave() { return __builtin_amdgcn_readfirstl
 // What the sorted keys stand for: ids (PlainKeys), or one field's column after the other, each key an offset in its
 // field's rows (FieldKeys, elr_dedup_plan_fields), where a column's first position is a head whatever its key.
 struct PlainKeys {
+  uint64_t lim;   // as in key_of; the key lim stands for ids that are no row: INT64_MAX, past every row
   template <typename Key>
-  __device__ __forceinline__ int64_t id(Key k, int64_t) const { return (int64_t)k; }
+  __device__ __forceinline__ int64_t id(Key k, int64_t) const {
+    return lim && (uint64_t)k == lim ? INT64_MAX : (int64_t)k;
+  }
   __device__ __forceinline__ bool starts(int64_t i) const { return i == 0; }
 };
 constexpr int kFieldMax = 128;   // fields per batch (the bounds travel as a kernel argument)
@@ -750,7 +765,8 @@ __global__ __launch_bounds__(kFieldThreads) void k_field_sort(const uint32_t* __
 constexpr int kSmallItems = 8;
 constexpr int64_t kSmallPlan = kFieldThreads * kSmallItems;
 template <typename Key, int ITEMS>
-__global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __restrict__ ids, int n, int passes, int rb,
+__global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __restrict__ ids, int n,
+                                                              PlainKeys keys, int passes, int rb,
                                                               int32_t* __restrict__ svals, int64_t* __restrict__ d_tot,
                                                               int64_t* __restrict__ n_unique,
                                                               int64_t* __restrict__ uniq,
@@ -768,7 +784,7 @@ __global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __r
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     const int j = (w * ITEMS + r) * 64 + lane;
-    kk[r] = (Key)ids[j < n ? j : 0];
+    kk[r] = key_of<Key>(ids[j < n ? j : 0], keys.lim);
   }
   if (t == 0) ecnt = hcnt = 0;
   const uint16_t* vfin = block_sort<Key, ITEMS>(s, kk, n, passes, rb);
@@ -808,7 +824,7 @@ __global__ __launch_bounds__(kFieldThreads) void k_small_plan(const int64_t* __r
       svals[j] = o;
       if (inverse) inverse[o] = u;
       if (head) {
-        uniq[u] = (int64_t)kk[r];
+        uniq[u] = keys.id(kk[r], j);
         seg_start[u] = j;
         seg_occ0[u] = o;
         if (hot_list) {
@@ -1486,35 +1502,58 @@ inline int sort_passes(int key_bits) {
   return passes;
 }
 
+// The low bits of a key that the radix passes of a key_bits-bit sort compare (at least key_bits).
+inline int sort_cover(int key_bits) {
+  int passes, rb;
+  sort_plan(key_bits, key_bits <= 32 ? max_digit_bits<uint32_t>() : max_digit_bits<uint64_t>(), passes, rb);
+  return passes * rb < 64 ? passes * rb : 64;
+}
+
+// Smallest b with bound < 2^b (at most 63): keys of b bits hold the ids in [0, bound) and at least one key more.  Only
+// a bound that is a power of two takes a bit for it, and only 2^10, 2^20 and 2^30 a pass (100,000 ids of width 32: 83 us
+// per update with 2^20 rows, 73 with 1,000,000).
+inline int bits_over(int64_t bound) {
+  int b = 1;
+  while (b < 63 && (int64_t(1) << b) <= bound) ++b;
+  return b;
+}
+
+// key_of's limit for ids of [0, bound) sorted with key_bits >= bits_over(bound): the highest key that the sort compares
+// whole (at least bound).  Ids between bound and it keep their own keys.
+inline uint64_t key_lim(int key_bits) {
+  const int c = sort_cover(key_bits);
+  return c < 64 ? (uint64_t(1) << c) - 1 : uint64_t(1) << 63;
+}
+
 // One pass over RB-bit digit p of the keys: histogram, scan (or none: fold), stable scatter from buffer cur (the
 // caller's ids on the first pass) to buffer nxt.
 template <typename Key, int RB, int NT>
-static void radix_pass_nt(const int64_t* ids, int64_t n, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
+static void radix_pass_nt(const int64_t* ids, int64_t n, uint64_t lim, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
   const int64_t ntile = sort_tiles(n);
   const int shift = RB * p, fold = ntile <= kSortFoldTiles;
   const unsigned grid = (unsigned)ntile;
   constexpr int BINS = 1 << RB;
   constexpr unsigned kScanGrid = (unsigned)(BINS / (kHistScanThreads / 64));   // a wave per digit
   Key* kb[2] = {(Key*)S.keys[0], (Key*)S.keys[1]};
-  if (p == 0) k_radix_hist<int64_t, Key, RB, NT><<<grid, NT, 0, st>>>(ids, n, shift, S.hist, ntile, fold);
-  else k_radix_hist<Key, Key, RB, NT><<<grid, NT, 0, st>>>(kb[cur], n, shift, S.hist, ntile, fold);
+  if (p == 0) k_radix_hist<int64_t, Key, RB, NT><<<grid, NT, 0, st>>>(ids, n, lim, shift, S.hist, ntile, fold);
+  else k_radix_hist<Key, Key, RB, NT><<<grid, NT, 0, st>>>(kb[cur], n, 0, shift, S.hist, ntile, fold);
   if (!fold) k_radix_hist_scan<<<kScanGrid, kHistScanThreads, 0, st>>>(S.hist, ntile, BINS, S.dtot);
   if (p == 0)
-    k_radix_scatter<int64_t, Key, true, RB, NT><<<grid, NT, 0, st>>>(ids, nullptr, n, shift, S.hist, S.dtot, (int)ntile,
-                                                                      fold, kb[nxt], S.vals[nxt]);
+    k_radix_scatter<int64_t, Key, true, RB, NT><<<grid, NT, 0, st>>>(ids, nullptr, n, lim, shift, S.hist, S.dtot,
+                                                                      (int)ntile, fold, kb[nxt], S.vals[nxt]);
   else
-    k_radix_scatter<Key, Key, false, RB, NT><<<grid, NT, 0, st>>>(kb[cur], S.vals[cur], n, shift, S.hist, S.dtot,
+    k_radix_scatter<Key, Key, false, RB, NT><<<grid, NT, 0, st>>>(kb[cur], S.vals[cur], n, 0, shift, S.hist, S.dtot,
                                                                    (int)ntile, fold, kb[nxt], S.vals[nxt]);
 }
 template <typename Key, int RB>
-static void radix_pass(const int64_t* ids, int64_t n, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
-  if (n >= kSortBig) radix_pass_nt<Key, RB, kSortThreadsBig>(ids, n, p, cur, nxt, S, st);
-  else radix_pass_nt<Key, RB, kSortThreadsSmall>(ids, n, p, cur, nxt, S, st);
+static void radix_pass(const int64_t* ids, int64_t n, uint64_t lim, int p, int cur, int nxt, DedupScratch& S, hipStream_t st) {
+  if (n >= kSortBig) radix_pass_nt<Key, RB, kSortThreadsBig>(ids, n, lim, p, cur, nxt, S, st);
+  else radix_pass_nt<Key, RB, kSortThreadsSmall>(ids, n, lim, p, cur, nxt, S, st);
 }
 
 // Sort (ids, positions) by id; returns which buffer holds the result.
 template <typename Key>
-static int radix_sort(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, hipStream_t st) {
+static int radix_sort(const int64_t* ids, int64_t n, uint64_t lim, int key_bits, DedupScratch& S, hipStream_t st) {
   int passes, rb;
   sort_plan(key_bits, max_digit_bits<Key>(), passes, rb);
   int cur = 0;
@@ -1522,13 +1561,13 @@ static int radix_sort(const int64_t* ids, int64_t n, int key_bits, DedupScratch&
     const int nxt = p == 0 ? 0 : cur ^ 1;
     if constexpr (max_digit_bits<Key>() >= 10) {
       if (rb == 10) {
-        radix_pass<Key, 10>(ids, n, p, cur, nxt, S, st);
+        radix_pass<Key, 10>(ids, n, lim, p, cur, nxt, S, st);
         cur = nxt;
         continue;
       }
     }
-    if (rb == 9) radix_pass<Key, 9>(ids, n, p, cur, nxt, S, st);
-    else radix_pass<Key, 8>(ids, n, p, cur, nxt, S, st);
+    if (rb == 9) radix_pass<Key, 9>(ids, n, lim, p, cur, nxt, S, st);
+    else radix_pass<Key, 8>(ids, n, lim, p, cur, nxt, S, st);
     cur = nxt;
   }
   return cur;
@@ -1558,17 +1597,18 @@ static void seg_plan(const Keys& keys, const Key* sk, const int32_t* sv, int64_t
     seg_plan_items<Key, kSegItemsSmall, Keys>(keys, sk, sv, n, S, uniq, inverse, n_unique, sums, st);
 }
 
-// Sort, segment heads and partial-chunk plan; returns which buffer holds the sorted positions.
+// Sort, segment heads and partial-chunk plan; returns which buffer holds the sorted positions.  The one-launch plan
+// compares at least the bits that the radix passes do, so both paths keep the same ids together.
 template <typename Key>
-static int dedup_core(const int64_t* ids, int64_t n, int key_bits, DedupScratch& S, int64_t* uniq_out,
-                      int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
-  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
+static int dedup_core_t(const int64_t* ids, int64_t n, int key_bits, uint64_t lim, DedupScratch& S, int64_t* uniq,
+                        int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
+  const PlainKeys keys{lim};
   if (n <= kSmallPlan) {
     int passes, rb;
-    digits_for(key_bits, passes, rb);
+    digits_for(sort_cover(key_bits), passes, rb);
     const int cur = (sort_passes<Key>(key_bits) - 1) % 2;   // where the radix passes would leave the positions
     auto go = [&](auto kern) {
-      kern<<<1, kFieldThreads, 0, st>>>(ids, (int)n, passes, rb, S.vals[cur], S.d_tot, n_unique, uniq, S.seg_start,
+      kern<<<1, kFieldThreads, 0, st>>>(ids, (int)n, keys, passes, rb, S.vals[cur], S.d_tot, n_unique, uniq, S.seg_start,
                                         S.seg_occ0, inverse, win_shift_for(n) ? nullptr : S.chunk_off, S.chunk_seg,
                                         sums ? S.hot_list : nullptr, (int)(win_shift_for(n) ? kWinHot : kHotLen));
     };
@@ -1578,10 +1618,17 @@ static int dedup_core(const int64_t* ids, int64_t n, int key_bits, DedupScratch&
     else go(k_small_plan<Key, kSmallItems>);
     return cur;
   }
-  const int cur = radix_sort<Key>(ids, n, key_bits, S, st);
+  const int cur = radix_sort<Key>(ids, n, lim, key_bits, S, st);
   const Key* sk = (const Key*)S.keys[cur];
-  seg_plan<Key>(PlainKeys{}, sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
+  seg_plan<Key>(keys, sk, S.vals[cur], n, S, uniq, inverse, n_unique, sums, st);
   return cur;
+}
+
+static int dedup_core(const int64_t* ids, int64_t n, int key_bits, uint64_t lim, DedupScratch& S, int64_t* uniq_out,
+                      int64_t* inverse, int64_t* n_unique, bool sums, hipStream_t st) {
+  int64_t* uniq = uniq_out ? uniq_out : S.uniq;
+  return key_bits <= 32 ? dedup_core_t<uint32_t>(ids, n, key_bits, lim, S, uniq, inverse, n_unique, sums, st)
+                        : dedup_core_t<uint64_t>(ids, n, key_bits, lim, S, uniq, inverse, n_unique, sums, st);
 }
 
 template <int NQ>
@@ -1674,12 +1721,6 @@ static int seg_reduce_d(const float* grad, int64_t D, const int32_t* sv, DedupSc
   return ELR_OK;
 }
 
-inline int bits_for(int64_t bound) {  // smallest b with bound <= 2^b (keys in [0, bound))
-  int b = 1;
-  while (b < 63 && (int64_t(1) << b) < bound) ++b;
-  return b;
-}
-
 inline bool dedup_sizes_ok(int64_t n) { return n >= 0 && n < (int64_t(1) << 31); }
 
 }  // namespace elr
@@ -1698,8 +1739,7 @@ extern "C" int elr_unique(const int64_t* ids, int64_t n, int key_bits, int64_t* 
   DedupScratch S;
   if (scratch_bytes < dedup_scratch_bytes(n, 1, &S, scratch)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
-  if (key_bits <= 32) dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, false, st);
-  else dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, false, st);
+  dedup_core(ids, n, key_bits, 0, S, uniq, inverse, n_unique, false, st);
   return launch_status();
 }
 
@@ -1713,9 +1753,8 @@ extern "C" int elr_segment_sum(const float* grad, const int64_t* idx, int64_t n,
   DedupScratch S;
   if (scratch_bytes < dedup_scratch_bytes(n, D, &S, scratch)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
-  const int kb = bits_for(num_rows);
-  const int cur = kb <= 32 ? dedup_core<uint32_t>(idx, n, kb, S, nullptr, nullptr, nullptr, true, st)
-                           : dedup_core<uint64_t>(idx, n, kb, S, nullptr, nullptr, nullptr, true, st);
+  const int kb = bits_over(num_rows);
+  const int cur = dedup_core(idx, n, kb, key_lim(kb), S, nullptr, nullptr, nullptr, true, st);
   const AdamScalars none{};
   const int rc = seg_reduce_d<0>(grad, D, S.vals[cur], S, S.uniq, n, out, num_rows, none, st);
   return rc != ELR_OK ? rc : launch_status();
@@ -1732,9 +1771,8 @@ extern "C" int elr_adam_dedup(float* state, int64_t C, const int64_t* ids, const
   if (scratch_bytes < dedup_scratch_bytes(n, D, &S, scratch)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
   const AdamScalars s = make_scalars(sc);
-  const int kb = bits_for(C);
-  const int cur = kb <= 32 ? dedup_core<uint32_t>(ids, n, kb, S, nullptr, nullptr, nullptr, true, st)
-                           : dedup_core<uint64_t>(ids, n, kb, S, nullptr, nullptr, nullptr, true, st);
+  const int kb = bits_over(C);
+  const int cur = dedup_core(ids, n, kb, key_lim(kb), S, nullptr, nullptr, nullptr, true, st);
   const int rc = seg_reduce_d<1>(grad, D, S.vals[cur], S, S.uniq, n, state, C, s, st);
   return rc != ELR_OK ? rc : launch_status();
 }
@@ -1754,8 +1792,8 @@ extern "C" int64_t elr_dedup_plan_bytes(int64_t n, int64_t D) {
   return dedup_scratch_bytes(n, D, nullptr, nullptr);
 }
 
-extern "C" int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64_t* uniq, int64_t* inverse,
-                              int64_t* n_unique, void* plan, int64_t plan_bytes, int64_t D, void* stream) {
+static int dedup_plan(const int64_t* ids, int64_t n, int key_bits, uint64_t lim, int64_t* uniq, int64_t* inverse,
+                      int64_t* n_unique, void* plan, int64_t plan_bytes, int64_t D, void* stream) {
   using namespace elr;
   if (!dedup_sizes_ok(n) || key_bits < 1 || key_bits > 64 || D < 1) return ELR_EINVAL;
   if (n == 0) return ELR_OK;
@@ -1763,10 +1801,21 @@ extern "C" int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64
   DedupScratch S;
   if (plan_bytes < dedup_scratch_bytes(n, D, &S, plan)) return ELR_ECAPACITY;
   hipStream_t st = (hipStream_t)stream;
-  const int cur = key_bits <= 32 ? dedup_core<uint32_t>(ids, n, key_bits, S, uniq, inverse, n_unique, true, st)
-                                 : dedup_core<uint64_t>(ids, n, key_bits, S, uniq, inverse, n_unique, true, st);
+  const int cur = dedup_core(ids, n, key_bits, lim, S, uniq, inverse, n_unique, true, st);
   if (cur != plan_result_buffer(key_bits)) return ELR_EINVAL;
   return launch_status();
+}
+
+extern "C" int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64_t* uniq, int64_t* inverse,
+                              int64_t* n_unique, void* plan, int64_t plan_bytes, int64_t D, void* stream) {
+  return dedup_plan(ids, n, key_bits, 0, uniq, inverse, n_unique, plan, plan_bytes, D, stream);
+}
+
+extern "C" int elr_dedup_plan_bounded(const int64_t* ids, int64_t n, int64_t bound, int64_t* uniq, int64_t* inverse,
+                                      int64_t* n_unique, void* plan, int64_t plan_bytes, int64_t D, void* stream) {
+  if (bound < 0) return ELR_EINVAL;
+  const int kb = elr::bits_over(bound);
+  return dedup_plan(ids, n, kb, elr::key_lim(kb), uniq, inverse, n_unique, plan, plan_bytes, D, stream);
 }
 
 extern "C" int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t nfields, const int64_t* field_lo,
@@ -1780,11 +1829,11 @@ extern "C" int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t 
   if (field_lo[0] < 0) return ELR_EINVAL;
   for (int64_t c = 0; c < nfields; ++c)
     if (field_lo[c + 1] < field_lo[c]) return ELR_EINVAL;
-  if (nrows > kFieldRows || nfields > kFieldMax || n <= kAtenSmall)
-    return elr_dedup_plan(ids, n, key_bits, uniq, inverse, n_unique, plan, plan_bytes, D, stream);
-  for (int64_t c = 0; c < nfields; ++c)
-    if (field_lo[c + 1] - field_lo[c] > kFieldSpanMax)
-      return elr_dedup_plan(ids, n, key_bits, uniq, inverse, n_unique, plan, plan_bytes, D, stream);
+  bool general = nrows > kFieldRows || nfields > kFieldMax || n <= kAtenSmall;
+  for (int64_t c = 0; c < nfields; ++c) general = general || field_lo[c + 1] - field_lo[c] > kFieldSpanMax;
+  if (general)   // (key_bits that leave no key for an id past the last field: the ids as they are)
+    return dedup_plan(ids, n, key_bits, key_bits >= bits_over(field_lo[nfields]) ? key_lim(key_bits) : 0, uniq, inverse,
+                      n_unique, plan, plan_bytes, D, stream);
   if (!ids || !uniq || !n_unique || !plan) return ELR_EINVAL;
   DedupScratch S;
   if (plan_bytes < dedup_scratch_bytes(n, D, &S, plan)) return ELR_ECAPACITY;

@@ -99,7 +99,7 @@ def field_bounds(lo):
 
 def unique_plan(ids, D, bound=None, fields=None):
     """unique(ids) without the inverse, keeping the sort as a plan for segment_sum_plan over gradients of width D:
-    returns (u, plan).  fields: see unique_plan_async."""
+    returns (u, plan).  With `bound`, ids may lie outside [0, bound): see unique_plan_async.  fields: see there too."""
     u, plan, nu = unique_plan_async(ids, D, bound, fields=fields)
     if nu is not None:
         plan.U = int(nu)
@@ -119,6 +119,8 @@ def plan_bytes(n, D):
 def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None, stream=None):
     """unique_plan without reading the unique count: returns (u_full, plan, nu) with u_full [n] whose first nu
     entries are the unique ids, nu the count on the device (None when n == 0).  Set plan.U once nu is known.
+    With `bound`, an id outside [0, bound) is kept apart from the rows in [0, bound) and comes out in u as itself or as
+    2^63 - 1: a row out of range, which adam_dedup_plan and segment_sum_plan (perm) skip.
     nu_out (int64 [1] on the device, optional): where the count goes, else a new tensor.
     out (optional): (buf, u, nu) to write into instead of new tensors -- uint8 buf of at least plan_bytes(n, D)
     bytes, int64 u of at least n elements, int64 nu [1] (nu_out, if given, takes its place); the caller keeps them
@@ -139,7 +141,11 @@ def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None, st
     plan.buf, plan.nbytes, plan.key_bits = None, 0, 1
     if n == 0:
         return torch.empty(0, dtype=I64, device=dev), plan, None
-    plan.key_bits = _key_bits(flat, bound)
+    if bound is not None:
+        bound = min(max(int(bound), 0), (1 << 63) - 1)
+        plan.key_bits = _bits(bound + 1)   # a key more than the rows': ids outside [0, bound) have one of their own
+    else:
+        plan.key_bits = _key_bits(flat, None)
     nbytes = plan_bytes(n, D)
     if out is not None:
         buf, u, nu0 = out
@@ -166,8 +172,12 @@ def unique_plan_async(ids, D, bound=None, nu_out=None, out=None, fields=None, st
                                                   st)
             _lib.check(rc, 'elr_dedup_plan_fields')
             return u, plan, nu
-        rc = _lib.lib().elr_dedup_plan(_lib.ptr(flat), n, plan.key_bits, _lib.ptr(u), None, _lib.ptr(nu),
-                                       _lib.ptr(plan.buf), nbytes, int(D), st)
+        if bound is not None:
+            rc = _lib.lib().elr_dedup_plan_bounded(_lib.ptr(flat), n, bound, _lib.ptr(u), None, _lib.ptr(nu),
+                                                   _lib.ptr(plan.buf), nbytes, int(D), st)
+        else:
+            rc = _lib.lib().elr_dedup_plan(_lib.ptr(flat), n, plan.key_bits, _lib.ptr(u), None, _lib.ptr(nu),
+                                           _lib.ptr(plan.buf), nbytes, int(D), st)
     _lib.check(rc, 'elr_dedup_plan')
     return u, plan, nu
 

@@ -231,14 +231,14 @@ int elr_unique(const int64_t* ids, int64_t n, int key_bits, int64_t* uniq, int64
                void* scratch, int64_t scratch_bytes, void* stream);
 
 /* Replaces: aten.embedding_dense_backward(grad, inv, num_rows, -1, False) at srm2/train.py:429.  out[k] = sum of
- * grad[i] (fp32 [n, D]) over i with idx[i] == k (idx int64 [n] in [0, num_rows)), in the order above; rows of out
- * without an index are not written (the caller zero-fills).  D <= 512. */
+ * grad[i] (fp32 [n, D]) over i with idx[i] == k (idx int64 [n]; an index outside [0, num_rows) is skipped), in the
+ * order above; rows of out without an index are not written (the caller zero-fills).  D <= 512. */
 int elr_segment_sum(const float* grad, const int64_t* idx, int64_t n, int64_t D, int64_t num_rows, float* out,
                     void* scratch, int64_t scratch_bytes, void* stream);
 
 /* Duplicate-id row-sparse Adam (config C3; the dedup of srm2/train.py:352 and 429 followed by srm2/ops.py:59-67
- * gpu_adam on the unique rows): state fp32 [C,3,D]; ids int64 [n] in [0, C), repeats allowed; grad fp32 [n,D].
- * Each unique id gets one Adam step (scalars sc) with the sum of its gradients.  D <= 512. */
+ * gpu_adam on the unique rows): state fp32 [C,3,D]; ids int64 [n], repeats allowed; grad fp32 [n,D].  Each unique id
+ * in [0, C) gets one Adam step (scalars sc) with the sum of its gradients; any other id is skipped.  D <= 512. */
 int elr_adam_dedup(float* state, int64_t C, const int64_t* ids, const float* grad, int64_t n, int64_t D,
                    const float sc[8], void* scratch, int64_t scratch_bytes, void* stream);
 
@@ -263,6 +263,12 @@ int elr_adam_dedup_noalloc(float* state, int64_t C, const int64_t* ids, const fl
 int64_t elr_dedup_plan_bytes(int64_t n, int64_t D);
 int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64_t* uniq, int64_t* inverse, int64_t* n_unique,
                    void* plan, int64_t plan_bytes, int64_t D, void* stream);
+/* elr_dedup_plan for ids of [0, bound) that may hold others: an id outside [0, bound) never shares a segment with a row
+ * in [0, bound) nor splits one, and comes out in uniq as itself or as INT64_MAX, a row out of range for the caller either
+ * way.  The later calls over the plan take key_bits = the smallest b with bound < 2^b (at most 63).  ELR_EINVAL for
+ * bound < 0. */
+int elr_dedup_plan_bounded(const int64_t* ids, int64_t n, int64_t bound, int64_t* uniq, int64_t* inverse,
+                           int64_t* n_unique, void* plan, int64_t plan_bytes, int64_t D, void* stream);
 /* elr_dedup_plan for a batch laid out by field, as the reference's one-hot batches are (srm2/train.py:187-214:
  * global id = local id + the field's table offset, flattened in (sample, field) order): ids [nrows * nfields],
  * field c of sample i at ids[i * nfields + c], and field c's ids in [field_lo[c], field_lo[c + 1]) (field_lo: host
@@ -273,7 +279,9 @@ int elr_dedup_plan(const int64_t* ids, int64_t n, int key_bits, int64_t* uniq, i
  * chunks lie aside, which no result depends on).  An id outside its
  * field's rows breaks that contract: it comes out as -1 in uniq, a row out of range for the caller.  Shapes the
  * per-field sort does not take (nrows > 16,384, nfields > 128, nrows * nfields <= 3,072, a field of more than
- * 2^31 - 2 rows) go to elr_dedup_plan with the same arguments.  ELR_EINVAL for bounds that are not ascending. */
+ * 2^31 - 2 rows) take the sort of elr_dedup_plan with the same arguments; there an id outside [0, field_lo[nfields])
+ * comes out as elr_dedup_plan_bounded gives it, where field_lo[nfields] < 2^key_bits.  ELR_EINVAL for bounds that are
+ * not ascending. */
 int elr_dedup_plan_fields(const int64_t* ids, int64_t nrows, int64_t nfields, const int64_t* field_lo, int key_bits,
                           int64_t* uniq, int64_t* inverse, int64_t* n_unique, void* plan, int64_t plan_bytes,
                           int64_t D, void* stream);

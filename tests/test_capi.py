@@ -252,6 +252,9 @@ def test_planner_executor_dedup_argument_checks():
     assert L.elr_dedup_plan(None, 0, 20, None, None, None, None, 0, 8, None) == 0                   # n == 0
     assert L.elr_dedup_plan(fake, 10, 0, fake, None, fake, fake, 1 << 20, 8, None) == -1            # key bits
     assert L.elr_dedup_plan(fake, 10, 20, fake, None, fake, fake, 1, 8, None) == -3                 # plan too small
+    assert L.elr_dedup_plan_bounded(None, 0, 20, None, None, None, None, 0, 8, None) == 0           # n == 0
+    assert L.elr_dedup_plan_bounded(fake, 10, -1, fake, None, fake, fake, 1 << 20, 8, None) == -1   # bound
+    assert L.elr_dedup_plan_bounded(fake, 10, 20, fake, None, fake, fake, 1, 8, None) == -3         # plan too small
     lo = (ctypes.c_int64 * 4)(0, 100, 200, 300)
     F = L.elr_dedup_plan_fields
     assert F(None, 0, 3, lo, 20, None, None, None, None, 0, 8, None) == 0                           # n == 0

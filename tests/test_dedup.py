@@ -578,6 +578,51 @@ def test_gpu_dedup_edge_cases(dev):
         unique(torch.tensor([-1, 2], device=dev))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [300, 3073, 8192, 8193, 30_000])
+@pytest.mark.parametrize('C,D', [(10, 8), (200, 64), (4000, 30), (4096, 8), (16_384, 64), (65_536, 8), (300_000, 8),
+                                 (1 << 20, 8), (1 << 21, 8)])
+def test_gpu_ids_outside_the_table_leave_valid_rows_alone(dev, C, D, n):
+    """Ids that are no row, between the occurrences of valid ids whose low bits they share (-1, C, C + row, row + 2^b on
+    each side of the digits' widths and of 32 bits, the extremes of int64), in the one-launch plan and the radix passes and
+    in both summation orders: every valid row has the oracle's bits, the others are skipped -- adam_dedup, the same over
+    a plan, and the sums of embedding_dense_backward."""
+    from elara_amd.dedup import adam_dedup, adam_dedup_plan, embedding_dense_backward, unique_plan
+    print(f'[gpu-test] ids outside the table C={C} D={D} n={n}', flush=True)
+    rng = np.random.default_rng(C + n)
+    rows = np.unique(np.concatenate([[0, 5, C - 1, C // 2], rng.integers(0, C, 40)]))
+    ids = rng.choice(rows, n).astype(np.int64)
+    i64 = np.iinfo(np.int64)
+    out = rng.random(n) < 0.4
+    b = rng.choice([4, 8, 9, 10, 12, 14, 16, 18, 20, 21, 24, 32, 33, 48], n)
+    far = rng.choice(np.array([-1, -2, C, i64.min, i64.max, (1 << 32) - 1]), n)
+    alias = np.where(rng.random(n) < 0.5, ids + (np.int64(1) << b), np.where(rng.random(n) < 0.3, C + ids, far))
+    ids = np.where(out & ((alias < 0) | (alias >= C)), alias, ids)
+    g = (rng.standard_normal((n, D)) * np.exp2(rng.integers(-12, 12, (n, 1)))).astype(np.float32)
+    valid = (ids >= 0) & (ids < C)
+    assert valid.any() and not valid.all()
+    u, s, _ = O.segment_sum(np.where(valid, ids, C), g)     # (the others: one id of their own, dropped here)
+    u, s = u[:-1], s[:-1]
+    state = (rng.standard_normal((u.size, 3, D)) * 0.05).astype(np.float32)
+    state[:, 2] **= 2
+    ud, idd, gd = torch.from_numpy(u).to(dev), torch.from_numpy(ids).to(dev), torch.from_numpy(g).to(dev)
+    a = torch.full((C, 3, D), 0.5, device=dev)
+    a[ud] = torch.from_numpy(state).to(dev)
+    b, idle = a.clone(), torch.ones(C, dtype=torch.bool, device=dev)
+    idle[ud] = False
+    O.cpu_adam(state, np.arange(u.size), s, O.adam_scalars(*HP, 3), 2)
+    adam_dedup(a, idd, gd, *HP, 3)
+    pu, plan = unique_plan(idd, D, C)
+    adam_dedup_plan(b, pu, gd, plan, *HP, 3)
+    sums = embedding_dense_backward(gd, idd, C)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(a[ud].cpu().numpy()), bits(state)) and bool((a[idle] == 0.5).all())
+    assert torch.equal(a, b)
+    assert np.array_equal(bits(sums[ud].cpu().numpy()), bits(s)) and not bool(sums[idle].any())
+    got = pu.cpu().numpy()
+    assert np.array_equal(got[(got >= 0) & (got < C)], u) and (np.diff(got) > 0).all()
+
+
 class _OraclePipe:
     """The CPU side of a long full-size run: each step's oracle work split into a part that is independent per step
     (`prep`, run by a pool of threads, several steps at once; the oracle's C calls release the GIL) and the part
