@@ -1041,11 +1041,25 @@ __device__ __forceinline__ void SegFinalSub<LPR, NC, MODE, WIN>::emit(int64_t ro
   }
 }
 
+// A staging area's rows are loaded into registers while the one before is added, the row indices of the one after (WIN)
+// with them, and the adding lanes read UN rows from LDS before the first addition: a row costs neither a round trip to
+// memory nor one to LDS.  3,000 occurrences of one id in the windowed order, whole update: 413 -> 264 us at width 48,
+// 489 -> 286 at 128, 1,262 -> 468 at 512 (each row read from LDS on its own, each staging area loaded between two
+// barriers), against 344, 417 and 905 for one wave that loads 8 rows together.
 template <int LPR, int NC, int MODE, bool WIN>
 __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
+  constexpr int NL = kSubStage / 4 / 256;   // chunks of a staging area per thread
+  constexpr int UN = 8 / NC;
   __shared__ f32x4 stage[kSubStage / 4];
   __shared__ int32_t win[WIN ? kSubStage / 4 : 1];   // windowed: the staged rows' windows
   const int t = threadIdx.x, nchunk = (int)(D / 4), per = (kSubStage / 4) / nchunk;
+  int rr[NL], cc[NL];   // this thread's chunks of a staging area: row and chunk (rr == per: none)
+#pragma unroll
+  for (int e = 0; e < NL; ++e) {
+    const int q = t + e * 256;
+    rr[e] = q / nchunk < per ? q / nchunk : per;
+    cc[e] = q % nchunk;
+  }
   const int64_t nh = *d_hot;
   for (int64_t h = block; h < nh; h += hot_blocks) {
     const int64_t u = hot_list[h], s0 = seg_start[u], L = seg_start[u + 1] - s0;
@@ -1054,33 +1068,67 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
         WIN ? grad : parts + (int64_t)chunk_off[u] * kGroupsPerChunk * D);
     RowFrag<4 * NC> tot = frag_zero<4 * NC>(), acc = tot;
     int32_t prev = -1;
+    int32_t ix[NL];    // rows of the staging area loaded next (rows past the last: the last)
+    int32_t wn[NL];    // windows of the rows in x
+    f32x4 x[NL];
+    auto index = [&](int64_t r0) {
+#pragma unroll
+      for (int e = 0; e < NL; ++e) {
+        const int64_t r = r0 + rr[e] < nr ? r0 + rr[e] : nr - 1;
+        ix[e] = WIN ? sv[s0 + r] : (int32_t)r;
+      }
+    };
+    auto load = [&] {
+#pragma unroll
+      for (int e = 0; e < NL; ++e) {
+        x[e] = src[(int64_t)ix[e] * nchunk + cc[e]];
+        wn[e] = ix[e] >> kAtenWinShift;
+      }
+    };
+    index(0);
+    load();
+    index(per);
     for (int64_t r0 = 0; r0 < nr; r0 += per) {
       const int m = (int)(nr - r0 < per ? nr - r0 : per);
       __syncthreads();
-      for (int q = t; q < m * nchunk; q += 256) {
-        const int r = q / nchunk;
-        const int64_t row = WIN ? (int64_t)sv[s0 + r0 + r] : r0 + r;
-        if (WIN && q - r * nchunk == 0) win[r] = (int32_t)(row >> kAtenWinShift);
-        stage[q] = src[row * nchunk + (q - r * nchunk)];
-      }
+#pragma unroll
+      for (int e = 0; e < NL; ++e)
+        if (rr[e] < m) {
+          stage[rr[e] * nchunk + cc[e]] = x[e];
+          if (WIN && cc[e] == 0) win[rr[e]] = wn[e];
+        }
       __syncthreads();
+      if (r0 + per < nr) {   // (block-uniform)
+        load();
+        index(r0 + 2 * per);
+      }
       if (t < LPR) {
-        for (int r = 0; r < m; ++r) {
-          RowFrag<4 * NC> x;
+        for (int r = 0; r < m; r += UN) {
+          RowFrag<4 * NC> y[UN];
+          int32_t yw[UN];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            const f32x4 g = t + c * LPR < nchunk ? stage[r * nchunk + t + c * LPR] : f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int i = 0; i < UN; ++i) {
+            const int ri = r + i < m ? r + i : r;
+            yw[i] = WIN ? __builtin_amdgcn_readfirstlane(win[ri]) : 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) x.v[4 * c + j] = g[j];
+            for (int c = 0; c < NC; ++c) {
+              const f32x4 g = stage[ri * nchunk + (t + c * LPR < nchunk ? t + c * LPR : 0)];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) y[i].v[4 * c + j] = g[j];
+            }
           }
-          if (!WIN) {
-            frag_add<4 * NC>(tot, x);
-          } else if (win[r] != prev) {
-            if (prev >= 0) frag_add<4 * NC>(tot, acc);
-            acc = x;
-            prev = win[r];
-          } else {
-            frag_add<4 * NC>(acc, x);
+#pragma unroll
+          for (int i = 0; i < UN; ++i) {
+            if (r + i >= m) continue;
+            if (!WIN) {
+              frag_add<4 * NC>(tot, y[i]);
+            } else if (yw[i] != prev) {
+              if (prev >= 0) frag_add<4 * NC>(tot, acc);
+              acc = y[i];
+              prev = yw[i];
+            } else {
+              frag_add<4 * NC>(acc, y[i]);
+            }
           }
         }
       }

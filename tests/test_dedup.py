@@ -326,6 +326,28 @@ def test_gpu_segment_lengths_in_chunk_layout(dev, D, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('D', [4, 48, 64, 128, 256, 320, 512])
+@pytest.mark.parametrize('n,hot', [(66, 65), (3072, 3072), (3000, 1500), (20_000, 20_000), (20_000, 9_999)])
+def test_gpu_hot_ids_fill_the_staging_area_many_times(dev, D, n, hot):
+    """One id that holds all or half of a batch (8 to 1,024 rows per staging area by width, the last one partly filled, rows
+    added 8 or 4 at a time), both summation orders: sums bitwise ATen's on this GPU and the oracle's."""
+    from elara_amd.dedup import embedding_dense_backward
+    print(f'[gpu-test] hot id D={D} n={n} hot={hot}', flush=True)
+    rng = np.random.default_rng(n + D + hot)
+    ids = np.full(n, 3, np.int64)
+    ids[rng.choice(n, n - hot, replace=False)] = 100 + np.arange(n - hot)
+    g = (rng.standard_normal((n, D)) * np.exp2(rng.integers(-12, 12, (n, 1)))).astype(np.float32)
+    g[ids == 3, 0] = np.float32(-0.0)
+    U = 101 + n - hot
+    gd, idd = torch.from_numpy(g).to(dev), torch.from_numpy(ids).to(dev)
+    got = embedding_dense_backward(gd, idd, U)
+    aten = torch.ops.aten.embedding_dense_backward(gd, idd, U, -1, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got.cpu().numpy()), bits(full_sums(ids, g, U)))
+    assert np.array_equal(bits(got.cpu().numpy()), bits(aten.cpu().numpy()))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('n', [(1 << 22) + 1, 9_000, 530_000])
 def test_gpu_sort_and_segments_at_their_limits(dev, n):
     """The sort with its digit counts added up in the scatter (up to 128 tiles of 4,096) and from a scan launch, the
