@@ -8,6 +8,7 @@ import contextlib
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -238,15 +239,20 @@ _host = None
 
 
 def host():
-    """The native argument checks of the row ops (csrc/hostcall.cpp), bound to the loaded library."""
+    """The native argument checks of the row ops (csrc/hostcall.cpp), bound to the loaded library.  Without the module,
+    or with one built for another torch or Python, a warning says so once and the Python path takes every call."""
     global _host
     if _host is None:
         L = lib()
         try:
             from . import _hostcall as h
+            if h.TORCH != torch.__version__:
+                raise ImportError(f'built for torch {h.TORCH}, this is {torch.__version__}')
             h.bind(*(ctypes.cast(f, c_vp).value for f in (L.elr_adam_scalars, L.elr_adam_rows, L.elr_init_rows,
                                                           L.elr_replay_rows)))
-        except ImportError:
+        except ImportError as e:
+            warnings.warn(f'elara_amd._hostcall is not used (small row-op calls take several microseconds longer): {e}',
+                          stacklevel=3)
             h = _NoHost
         _host = h
     return _host

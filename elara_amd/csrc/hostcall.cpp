@@ -11,6 +11,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <cstring>
+
 #include <ATen/ops/empty.h>
 #include <c10/core/DefaultDtype.h>
 #include <c10/hip/HIPStream.h>
@@ -199,6 +201,8 @@ PyObject* replay(PyObject*, PyObject* const* a, Py_ssize_t na) {
   }
 }
 
+#define ELR_STR1(x) #x
+#define ELR_STR(x) ELR_STR1(x)
 #define ELR_FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f))
 PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, "Addresses of the library's entry points."},
                          {"adam", ELR_FAST(adam), METH_FASTCALL, "elr_adam_rows with gpu_adam's checks."},
@@ -209,8 +213,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, methods, 
 
 }  // namespace
 
+// The file's name carries neither version, and another Python's or torch's objects are laid out differently: the former is
+// refused here, the latter by the caller (elara_amd/_lib.py: host), both before any tensor is touched.
 PyMODINIT_FUNC PyInit__hostcall() {
+  constexpr const char built[] = ELR_STR(PY_MAJOR_VERSION) "." ELR_STR(PY_MINOR_VERSION) ".";
+  if (std::strncmp(Py_GetVersion(), built, sizeof built - 1) != 0) {
+    PyErr_Format(PyExc_ImportError, "_hostcall was built for Python %sx", built);
+    return nullptr;
+  }
   PyObject* m = PyModule_Create(&module);
-  if (m) PyModule_AddIntConstant(m, "NOT_TAKEN", kNotTaken);
+  if (m) {
+    PyModule_AddIntConstant(m, "NOT_TAKEN", kNotTaken);
+    PyModule_AddStringConstant(m, "TORCH", ELR_TORCH_VERSION);
+  }
   return m;
 }

@@ -30,6 +30,47 @@ def test_library_exports_every_declared_symbol():
     assert set(names) <= set(_lib.SIGNATURES), 'binding lacks a signature for a declared entry point'
 
 
+def test_library_is_built_where_the_host_module_cannot_be(monkeypatch, tmp_path):
+    """The host module's build failing leaves a linked library, no older module and a warning."""
+    import subprocess
+    from elara_amd import build
+    old = tmp_path / '_hostcall.so'
+    old.write_bytes(b'an older build')
+    monkeypatch.setattr(build, 'HERE', tmp_path)
+    monkeypatch.setattr(build, 'LIB', tmp_path / 'lib.so')
+    monkeypatch.setattr(build, 'HOST_LIB', old)
+    monkeypatch.setattr(build, '_compile', lambda src, obj: obj)
+
+    def tool(cmd, **kw):
+        out = Path(cmd[cmd.index('-o') + 1])
+        ok = cmd[0] == build.HIPCC
+        if ok:
+            out.write_bytes(b'linked')
+        return subprocess.CompletedProcess(cmd, 0 if ok else 1, '', '' if ok else 'g++: not found')
+    monkeypatch.setattr(build.subprocess, 'run', tool)
+    with pytest.warns(UserWarning, match='_hostcall.so was not built'):
+        assert build.build() == tmp_path / 'lib.so'
+    assert (tmp_path / 'lib.so').read_bytes() == b'linked' and not old.exists()
+
+
+@pytest.mark.parametrize('why', ['absent', 'another torch'])
+def test_host_module_fallback_says_so_once(monkeypatch, why):
+    import sys
+    import warnings
+    import torch
+    monkeypatch.setattr(_lib, '_host', None)
+    if why == 'absent':
+        monkeypatch.setitem(sys.modules, 'elara_amd._hostcall', None)
+        monkeypatch.delattr('elara_amd._hostcall', raising=False)
+    else:
+        monkeypatch.setattr(torch, '__version__', '0.0')
+    with pytest.warns(UserWarning, match='_hostcall is not used'):
+        assert _lib.host() is _lib._NoHost
+    with warnings.catch_warnings():
+        warnings.simplefilter('error')
+        assert _lib.host() is _lib._NoHost
+
+
 def test_struct_layouts_match_the_library():
     """Every ctypes mirror of a header struct has the size the library was compiled with (elr_abi_sizes)."""
     out = (ctypes.c_int64 * len(_lib.ABI_STRUCTS))()
