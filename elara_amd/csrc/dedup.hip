@@ -54,6 +54,8 @@ constexpr int kSegItemsBig = 8;
 constexpr int kSegItemsSmall = 4;
 constexpr int64_t kSegBig = int64_t(1) << 20;
 inline int seg_items_for(int64_t n) { return n >= kSegBig ? kSegItemsBig : kSegItemsSmall; }
+// LDS of a CU, and what a block's small shared arrays (scans, counters) take beside its large ones, at most.
+constexpr size_t kLdsBytes = 160 * 1024, kLdsSlack = 1024;
 constexpr int kRadixMaxBits = 10;   // passes take digits of 8, 9 or 10 bits (sort_plan)
 constexpr int kRadixMaxBins = 1 << kRadixMaxBits;
 constexpr int64_t kAtenSmall = 3072;                      // ATen's windowed path up to this many indices
@@ -206,6 +208,8 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ sr
   __shared__ uint16_t wc[NW][BINS];   // per wave: running count of digit d, then the count in earlier waves
   __shared__ Key lk[TILE];
   __shared__ int32_t lv[TILE];
+  static_assert(sizeof(bo) + sizeof(lbase) + sizeof(wc) + sizeof(lk) + sizeof(lv) + kLdsSlack <= kLdsBytes / 2,
+                "two blocks per CU");
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   const int64_t tile0 = (int64_t)blockIdx.x * TILE, base = tile0 + (int64_t)w * (ITEMS * 64);
   // the tile's items first, so that their loads overlap the digit bases' loads and scan
@@ -647,6 +651,7 @@ template <typename Key, int ITEMS>
 __device__ __forceinline__ const uint16_t* block_sort(BlockSort<Key, ITEMS>& s, Key (&kk)[ITEMS], int n, int passes,
                                                       int rb) {
   constexpr int NW = kFieldThreads / 64, WSPAN = ITEMS * 64;
+  static_assert(sizeof(BlockSort<Key, ITEMS>) + kLdsSlack <= kLdsBytes, "one block per CU");
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   const int nbins = 1 << rb;
   const uint32_t mask = (uint32_t)nbins - 1u;
@@ -1520,12 +1525,14 @@ inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void
   s.keys[1] = take(n * 8);
   s.vals[0] = (int32_t*)take(n * 4);
   s.vals[1] = (int32_t*)take(n * 4);
-  // the digit counts, then the segment tiles' counts; the digit totals
+  // the digit counts (the first half), then the segment tiles' counts; the digit totals (the first half).  The halves
+  // that nothing reads, and the unused region, keep every n's scratch size, and with it the largest n that
+  // elr_adam_dedup_noalloc takes, where it has been.
   s.hist = (int32_t*)take(kRadixMaxBins * ntile * 8);
   s.bsum = (int64_t*)(s.hist + kRadixMaxBins * ntile);
   s.bfirst = (int32_t*)(s.bsum + nblk);
   s.dtot = (int32_t*)take(kRadixMaxBins * 8);
-  o += al256(ntile * 8);   // unused: keeps the largest n of elr_adam_dedup_noalloc where it has been
+  o += al256(ntile * 8);   // unused
   s.d_tot = (int64_t*)take(3 * 8);
   s.uniq = (int64_t*)take(n * 8);
   s.seg_start = (int64_t*)take((n + 1) * 8);
@@ -1538,7 +1545,8 @@ inline int64_t dedup_scratch_bytes(int64_t n, int64_t D, DedupScratch* out, void
   return o;
 }
 
-// Widest digit of a sort with Key keys: 64-bit keys stop at 9 bits to keep the scatter's LDS tile within 64 KiB.
+// Widest digit of a sort with Key keys.  64-bit keys take 9 bits at most, the widest measured for them.  The scatter's LDS
+// with 1,024 threads: 72 KiB at 10 bits of 32-bit keys, 68 at 9 of 64, so two blocks fit a CU (its static_assert).
 template <typename Key>
 constexpr int max_digit_bits() { return sizeof(Key) == 8 ? 9 : kRadixMaxBits; }
 

@@ -206,8 +206,9 @@ __global__ __launch_bounds__(256) void k_replay_wpr(float* __restrict__ out, con
       const int ci = cnt[i];
       const int cc = ci < 0 ? 0 : (ci > K ? K : ci);
       // every used step indexes the table and every used log entry exists (branch-free).  Up to K = 4 a row without
-      // entries is held to 0 <= offset <= nlogs too, as packed logs give it: letting it pass with any offset, as the
-      // other kernels do, costs 2 of 117 us at 262,144 rows of width 128.
+      // entries is held to 0 <= offset <= nlogs too, as the entry point asks: letting it pass with any offset, as the
+      // other kernels do, costs 2 of 118 us at 262,144 rows of width 128 and K = 3 (by the count or by an offset of 0
+      // for it), 4 of 100 at K = 1 (by the count).
       int bad = (o[u] < 0) | (o[u] > nlogs - cc);
       if constexpr (K > 4) bad &= cc > 0;
 #pragma unroll

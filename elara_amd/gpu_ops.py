@@ -59,7 +59,8 @@ class ScalarTable:
 
 
 def replay_rows(rows, logs, offs, steps, cnt, D, K, seed, bound, table, out=None, events=None):
-    """rows int64 [n]; logs [sum(cnt), D] with row i's entries at offs[i]; steps int32 [n,K]; cnt int32 [n];
+    """rows int64 [n]; logs [sum(cnt), D] with row i's entries at offs[i] (0 <= offs[i] and offs[i] + cnt[i] <= len(logs) for
+    every row, also one without entries: a row that breaks this may be left unwritten); steps int32 [n,K]; cnt int32 [n];
     table: ScalarTable (or its [S,8] tensor) -> out [n,3,D].  Allocates `out` when None.  events: optional
     (start, stop) hipEvent_t handles (integers) that the launch itself records at the kernel's start and end
     (elr_replay_rows_timed); not recorded when n == 0."""

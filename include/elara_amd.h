@@ -103,7 +103,8 @@ int elr_init_rows(float* out, const int64_t* rows, int64_t n, int64_t D, uint32_
  * Replaces: srm2/gpu_ops.py:91-99 replay_rows / _replay (gpu_ops.py:51-79).  out[i] = init(rows[i]) followed by
  * Adam with gradient logs[offs[i] + k] and scalars table[steps[i*K + k]] for k < cnt[i].  1 <= K <= 8.
  *   out device fp32 [n,3,D]; rows int64 [n]; logs fp32 [nlogs,D]; offs int64 [n]; steps int32 [n,K];
- *   cnt int32 [n]; table fp32 [table_rows, 8]; recip fp64 [table_rows, 2] from elr_scalar_recip (copied to the
+ *   cnt int32 [n]; 0 <= offs[i] and offs[i] + cnt[i] <= nlogs for every row, also one without entries (a row that breaks
+ *   this may be skipped); table fp32 [table_rows, 8]; recip fp64 [table_rows, 2] from elr_scalar_recip (copied to the
  *   device), or NULL (then the kernel computes the reciprocals itself, at some cost).  All device pointers.
  * ------------------------------------------------------------------------------------------------------- */
 int elr_replay_rows(float* out, const int64_t* rows, const float* logs, int64_t nlogs, const int64_t* offs,

@@ -177,11 +177,13 @@ def test_gpu_unique_matches_torch(dev, case):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('key_bits', [1, 8, 9, 12, 17, 20, 24, 27, 30, 32, 33, 40, 63])
-@pytest.mark.parametrize('n', [70001, (1 << 18) - 1, (1 << 18) + 3, (1 << 21) + 3])
+@pytest.mark.parametrize('n', [1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 70001, (1 << 18) - 1, (1 << 18) + 3,
+                               (1 << 20) - 1, 1 << 20, (1 << 21) + 3])
 def test_gpu_unique_every_digit_width(dev, key_bits, n):
     """The sort takes 8-, 9- or 10-bit digits (fewer passes: 27-bit keys in 3 passes of 9 bits, 30-bit keys in 3 of
-    10); for each key width from the caller's bound, both tile sizes (either side of 2^18 ids) give torch.unique's
-    rows and inverse.  Ids are spread over the whole width, with duplicates and the extreme keys 0 and 2^b - 1."""
+    10) with 1,024 or 256 threads per tile (either side of 2^20 ids), and up to 8,192 ids one block of 1 to 8 keys per
+    thread; for each key width from the caller's bound, each gives torch.unique's rows and inverse.  Ids are spread over the
+    whole width, with duplicates and the extreme keys 0 and 2^b - 1."""
     from elara_amd.dedup import unique
     rng = np.random.default_rng(key_bits * 7 + n % 5)
     hi = (1 << key_bits) - 1
@@ -241,9 +243,9 @@ def test_gpu_embedding_backward_matches_aten(dev, n, U, D):
 @pytest.mark.gpu
 @pytest.mark.parametrize('n', [1 << 20, (1 << 20) + 1])
 def test_gpu_segment_block_offsets_both_ways(dev, n):
-    """The segment-head and chunk-plan launches take their block offsets by summing the earlier blocks' counts in
-    each block up to 256 blocks (2^20 ids in tiles of 4,096) and from a one-block scan launch above (one id more):
-    unique equals torch.unique and the sums equal ATen's embedding_dense_backward on both sides, with a hot id."""
+    """The segment launches at a batch that fills its tiles and at one id more (512 and 513 segment tiles, whose offsets
+    each block sums; the scan launch that gives them above 2,048 tiles: test_gpu_sort_and_segments_at_their_limits):
+    unique equals torch.unique and the sums equal ATen's embedding_dense_backward, with a hot id."""
     from elara_amd.dedup import embedding_dense_backward, unique
     U, D = 300_000, 64
     print(f'[gpu-test] block offsets n={n}', flush=True)
@@ -348,7 +350,7 @@ def test_gpu_hot_ids_fill_the_staging_area_many_times(dev, D, n, hot):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('n', [(1 << 22) + 1, 9_000, 530_000])
+@pytest.mark.parametrize('n', [1 << 22, (1 << 22) + 1, 9_000, 530_000])
 def test_gpu_sort_and_segments_at_their_limits(dev, n):
     """The sort with its digit counts added up in the scatter (up to 128 tiles of 4,096) and from a scan launch, the
     segment offsets from the blocks and (above 2,048 tiles) from a scan launch, an id that spans many tiles and ids
@@ -432,23 +434,26 @@ def field_case(case, rng):
     vocab = {'ragged': [1, 3, 511, 512, 513, 2**17, 70000],       # 5,000 rows: one hot id per tiny field
              'one_field': [2**20],                                  # 16,384 rows, one block
              'wide': [50] * 100,                                    # 100 rows x 100 fields
+             'two_keys': [400, 90000, 17],                          # 1,500 rows: 2 keys per thread
+             'four_keys': [400, 90000, 17],                         # 3,000 rows: 4 keys per thread
              'big_span': [2**31 - 2, 5, 40000],                     # keys of 31 bits: 4 passes
              'fallback_rows': [3000, 90000, 17],                    # 20,000 rows: the general sort
              'fallback_small': [100] * 26}[case]                    # 2,600 ids: ATen's windowed order
-    nrows = {'ragged': 5000, 'one_field': 16384, 'wide': 100, 'big_span': 12000, 'fallback_rows': 20000,
+    nrows = {'ragged': 5000, 'one_field': 16384, 'wide': 100, 'two_keys': 1500, 'four_keys': 3000, 'big_span': 12000, 'fallback_rows': 20000,
              'fallback_small': 100}[case]
     z = synth.ZipfFields(vocab, 1.1, seed=int(rng.integers(1 << 30)))
     return z.draw(rng, nrows), np.append(z.offsets, z.offsets[-1] + z.vocab[-1])
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('case', ['c5', 'ragged', 'one_field', 'wide', 'big_span', 'fallback_rows', 'fallback_small'])
+@pytest.mark.parametrize('case', ['c5', 'ragged', 'one_field', 'wide', 'two_keys', 'four_keys', 'big_span', 'fallback_rows',
+                                  'fallback_small'])
 def test_gpu_dedup_plan_fields_matches_general(dev, case):
     """A batch laid out by field, sorted per field (elr_dedup_plan_fields): the unique ids, the inverse and the
     segment sums over its plan are bitwise those of the general sort's plan and the oracle's; the unique count is
     the same.  Covers both result buffers of the plan (27- and 18-bit bounds), fields of one row (a hot segment of
-    every occurrence), digit widths at 2^9 +- 1, 31-bit keys, a hundred fields of 100 rows, and the shapes that go to
-    the general sort."""
+    every occurrence), digit widths at 2^9 +- 1, 31-bit keys, a hundred fields of 100 rows, each number of keys per
+    thread (1, 2, 4, 8, 16), and the shapes that go to the general sort."""
     import ctypes
     from elara_amd import _lib
     from elara_amd.dedup import field_bounds, plan_bytes, segment_sum_plan, unique_plan_async
