@@ -192,8 +192,10 @@ __device__ __forceinline__ void bins_excl_scan(const int (&x)[BPT], Put&& put) {
 // 64 scattered ones.  A digit's first position for this tile: the exclusive scan of the digit totals plus the
 // earlier tiles' counts, both from the scan launch (offs, dtot) or, with fold, summed here from the tile-major
 // histograms.
+// (256-thread blocks of 32-bit keys: four waves per SIMD, which their LDS allows, asked of the register allocator too; the
+// first pass otherwise takes 129 registers and three waves, 32 us against 27 at 3.4M keys)
 template <typename Src, typename Key, bool FIRST, int RB, int NT>
-__global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ src_keys,
+__global__ __launch_bounds__(NT, NT == kSortThreadsBig && sizeof(Key) == 4 ? 4 : 1) void k_radix_scatter(const Src* __restrict__ src_keys,
                                                                 const int32_t* __restrict__ src_vals, int64_t n,
                                                                 uint64_t lim, int shift, const int32_t* __restrict__ offs,
                                                                 const int32_t* __restrict__ dtot, int ntile, int fold,
@@ -212,15 +214,15 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ sr
                 "two blocks per CU");
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   const int64_t tile0 = (int64_t)blockIdx.x * TILE, base = tile0 + (int64_t)w * (ITEMS * 64);
-  // the tile's items first, so that their loads overlap the digit bases' loads and scan
-  Key kk[ITEMS];
+  // the tile's items first, so that their loads overlap the digit bases' loads and scan (the ids become keys after it: a
+  // use before it would wait for them)
+  Src in[ITEMS];
   int32_t vv[ITEMS];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     const int64_t pos = base + (int64_t)r * 64 + lane;
     const bool valid = pos < n;
-    const Src x = valid ? src_keys[pos] : (Src)0;
-    kk[r] = FIRST ? key_of<Key>((int64_t)x, lim) : (Key)x;
+    in[r] = valid ? src_keys[pos] : (Src)0;
     vv[r] = valid ? (FIRST ? (int32_t)pos : src_vals[pos]) : 0;
   }
   const bool own = t * BPT < BINS;   // this thread's digits
@@ -259,6 +261,9 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(const Src* __restrict__ sr
   });
   for (int q = t; q < NW * BINS / 2; q += NT) reinterpret_cast<uint32_t*>(&wc[0][0])[q] = 0;
   __syncthreads();
+  Key kk[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) kk[r] = FIRST ? key_of<Key>((int64_t)in[r], lim) : (Key)in[r];
   int rk[ITEMS];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
@@ -1057,6 +1062,8 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
   constexpr int UN = 8 / NC;
   __shared__ f32x4 stage[kSubStage / 4];
   __shared__ int32_t win[WIN ? kSubStage / 4 : 1];   // windowed: the staged rows' windows
+  const int64_t nh = *d_hot;
+  if (block >= nh) return;
   const int t = threadIdx.x, nchunk = (int)(D / 4), per = (kSubStage / 4) / nchunk;
   int rr[NL], cc[NL];   // this thread's chunks of a staging area: row and chunk (rr == per: none)
 #pragma unroll
@@ -1065,7 +1072,6 @@ __device__ void SegFinalSub<LPR, NC, MODE, WIN>::hot(int64_t block) const {
     rr[e] = q / nchunk < per ? q / nchunk : per;
     cc[e] = q % nchunk;
   }
-  const int64_t nh = *d_hot;
   for (int64_t h = block; h < nh; h += hot_blocks) {
     const int64_t u = hot_list[h], s0 = seg_start[u], L = seg_start[u + 1] - s0;
     const int64_t nr = WIN ? L : (L + kAtenGroup - 1) / kAtenGroup;   // rows to add: gradients, or run sums
