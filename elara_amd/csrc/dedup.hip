@@ -36,8 +36,9 @@
 namespace elr {
 
 // A sort tile is 4,096 keys: 1,024 threads with 4 keys each below kSortBig keys, where a tile's chain of ranking rounds
-// and LDS passes is what a launch takes (the scatters of 426k keys 9 us against 13.5 with 256 threads of 16 keys), and
-// 256 threads with 16 keys each from there, where several tiles per CU hide it (3.4M keys: 26 us against 36).
+// and LDS passes is what a launch takes (a pass of 426k keys, the digit counts summed as below: 18 us of histogram and
+// scatter, against 25 in three launches with 256 threads of 16 keys), and 256 threads with 16 keys each from there, where
+// several tiles per CU hide it (scatters of 3.4M keys: 26 us against 36).
 constexpr int kSortTile = 4096;
 constexpr int kSortThreadsSmall = 1024;
 constexpr int kSortThreadsBig = 256;
@@ -49,7 +50,8 @@ inline int64_t sort_tiles(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
 constexpr int64_t kSortFoldTiles = 128;
 static_assert(kSortFoldTiles * kSortTile <= kSortBig, "the scatters that sum the counts have 1,024 threads");
 // Rounds of a segment tile (k_seg_count, k_seg_apply): 8 from 2^20 positions, 4 below, so that a small batch still
-// spreads over the chip (426k positions: 8 us against 19 with 16 rounds; 3.4M: 27 us with 8 rounds, 29 with 16).
+// spreads over the chip (k_seg_count and k_seg_apply of 426k positions: 15 us against 20 with 16 rounds; of 3.4M: 33 with 8
+// rounds, 34 with 16).
 constexpr int kSegItemsBig = 8;
 constexpr int kSegItemsSmall = 4;
 constexpr int64_t kSegBig = int64_t(1) << 20;
@@ -460,8 +462,8 @@ __device__ __forceinline__ int part_chunks(int64_t L) {
 // A segment's length, which decides its chunks, is the distance to the next head: in its round's mask, in a later
 // round's or wave's, or in a later tile (bfirst).  The work items of a block's chunks are reserved with one atomic
 // add, so their order over the segments is not fixed; no sum depends on it (each group sum has its own parts row).
-// One launch in place of three (heads with a block scan per round, chunk counts, chunk plan): 28 us against 20 + 8 +
-// 20 and two scan launches of 4.5 at config C3's 3.4M positions, 10 against 18 + 8 + 21 at C5's 426k.
+// One launch in place of three (heads with a block scan per round, chunk counts, chunk plan): 33 us against 20 + 8 +
+// 24 and two scan launches of 4.6 at config C3's 3.4M positions, 11 against 16 + 7 + 23 at C5's 426k.
 template <typename Key, int ITEMS, class Keys>
 __global__ __launch_bounds__(kSegBlock) void k_seg_apply(Keys keys, const Key* __restrict__ sk,
                                                          const int32_t* __restrict__ sv, int64_t n, const int64_t* __restrict__ bcnt, int scanned,
@@ -770,7 +772,7 @@ __global__ __launch_bounds__(kFieldThreads) void k_field_sort(const uint32_t* __
 // ballots, the inverse, the hot segments and the partial-chunk plan -- what the radix passes, k_seg_count and
 // k_seg_apply leave, in one launch.  Against the general path's ten launches of 2 to 5 us each, every one waiting for
 // the one before, one block's passes over LDS are the shorter chain: 12.8 us at 2,600 ids, and the whole update of a
-// batch of 2,600 36.4 -> 17.8 us.  The line: whole updates of 7,800 ids 40.0 -> 35.1 and of 8,000 ids 58 -> 43 us by
+// batch of 2,600 36.4 -> 18.0 us.  The line: whole updates of 7,800 ids 40.0 -> 35.1 and of 8,000 ids 58 -> 43 us by
 // this kernel, its time growing with the ids while the general path's barely does.
 constexpr int kSmallItems = 8;
 constexpr int64_t kSmallPlan = kFieldThreads * kSmallItems;
@@ -1005,9 +1007,8 @@ __global__ __launch_bounds__(256) void k_seg_final(const float* __restrict__ gra
 // metadata; its gradient row and state), and a longer one two more per kSubRows occurrences.  The first hot_blocks
 // blocks take the segments of hot_list, one each at a time: the whole block loads the run sums (windowed: the
 // gradients) into LDS, kSubStage floats of them, and one group adds them in order.  Against a wave per segment with
-// 4 bytes a lane: 26 us
-// against 37 at 107k occurrences, 40k segments of width 48 (most of it the dependent round trips of the 60-occurrence
-// segments: 12 without them).
+// 4 bytes a lane: 24 us against 37 at 107k occurrences, 40k segments of width 48 (most of it the dependent round trips of the
+// 60-occurrence segments: 12 without them).
 template <int NC>
 constexpr int kSubRows = NC == 1 ? kAtenGroup : kAtenGroup / 2;
 constexpr int kSubStage = 4096;   // floats: 16 KB, so that LDS leaves the wave count alone
